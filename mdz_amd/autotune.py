@@ -35,7 +35,7 @@ import mdz_amd as M
 from mdz_amd import workloads as WL
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-NWORDS = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32)
+NWORDS = (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32)
 PROBE_W, PROBE_H = 1024, 512
 
 

@@ -21,7 +21,7 @@ LIB = os.path.join(HERE, "libmdzg.so")
 
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 MP_PREFIX = os.environ.get("MDZG_MP_PREFIX", "/opt/conda")
-NWORDS = (1, 2, 3, 4, 6, 8, 12, 16, 24, 32)
+NWORDS = (1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32)
 
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -1,7 +1,7 @@
 /*
  * launch.hip -- kernel table and launch wrappers called by the C host runtime.
  *
- * Kernel id: 0 = FP64; 1 + 2*i + full for the RN kernels of word count
+ * Kernel id: 0 = FP64; MDZG_RN_KID[i] + full for the RN kernels of word count
  * MDZG_NWORDS[i] (full = the tile precision is exactly 32N bits);
  * MDZG_KID_GMP0 + j for the GMP-path kernels of storage bucket j.
  */
@@ -17,11 +17,17 @@ void mdzg_kget_rn1(int, const void**, const void**, const void**);
 void mdzg_kget_rn2(int, const void**, const void**, const void**);
 void mdzg_kget_rn3(int, const void**, const void**, const void**);
 void mdzg_kget_rn4(int, const void**, const void**, const void**);
+void mdzg_kget_rn5(int, const void**, const void**, const void**);
 void mdzg_kget_rn6(int, const void**, const void**, const void**);
+void mdzg_kget_rn7(int, const void**, const void**, const void**);
 void mdzg_kget_rn8(int, const void**, const void**, const void**);
+void mdzg_kget_rn10(int, const void**, const void**, const void**);
 void mdzg_kget_rn12(int, const void**, const void**, const void**);
+void mdzg_kget_rn14(int, const void**, const void**, const void**);
 void mdzg_kget_rn16(int, const void**, const void**, const void**);
+void mdzg_kget_rn20(int, const void**, const void**, const void**);
 void mdzg_kget_rn24(int, const void**, const void**, const void**);
+void mdzg_kget_rn28(int, const void**, const void**, const void**);
 void mdzg_kget_rn32(int, const void**, const void**, const void**);
 void mdzg_kget_gmp(int bucket, const void**, const void**, const void**);
 const void* mdzg_kprobe_rn4(void);
@@ -30,9 +36,21 @@ const void* mdzg_kprobe_rn32(void);
 
 typedef void (*kget_fn)(int, const void**, const void**, const void**);
 static const kget_fn kget_rn[MDZG_NCLASS_N] = {
-    mdzg_kget_rn1, mdzg_kget_rn2, mdzg_kget_rn3, mdzg_kget_rn4, mdzg_kget_rn6,
-    mdzg_kget_rn8, mdzg_kget_rn12, mdzg_kget_rn16, mdzg_kget_rn24, mdzg_kget_rn32,
+    mdzg_kget_rn1,  mdzg_kget_rn2,  mdzg_kget_rn3,  mdzg_kget_rn4,
+    mdzg_kget_rn5,  mdzg_kget_rn6,  mdzg_kget_rn7,  mdzg_kget_rn8,
+    mdzg_kget_rn10, mdzg_kget_rn12, mdzg_kget_rn14, mdzg_kget_rn16,
+    mdzg_kget_rn20, mdzg_kget_rn24, mdzg_kget_rn28, mdzg_kget_rn32,
 };
+static const int rn_kid[MDZG_NCLASS_N] = MDZG_RN_KID_INIT;
+
+/* RN class of an RN kernel id */
+static int class_of_kid(int kid)
+{
+    int i = 0;
+    while (i < MDZG_NCLASS_N - 1 && kid != rn_kid[i] && kid != rn_kid[i] + 1)
+        ++i;
+    return i;
+}
 
 /* form: 0 = per-tile, 1 = persistent, 2 = resumable slice */
 static void lookup(int kid, int form, const void** f)
@@ -42,10 +60,10 @@ static void lookup(int kid, int form, const void** f)
     const void* sl = nullptr;
     if (kid == 0)
         mdzg_kget_fp64(&t, &p, &sl);
-    else if (kid >= MDZG_KID_GMP0)
+    else if (kid >= MDZG_KID_GMP0 && kid < MDZG_KID_GMP0 + MDZG_NGMP)
         mdzg_kget_gmp(kid - MDZG_KID_GMP0, &t, &p, &sl);
     else
-        kget_rn[(kid - 1) >> 1]((kid - 1) & 1, &t, &p, &sl);
+        kget_rn[class_of_kid(kid)]((kid - 1) & 1, &t, &p, &sl);
     *f = form == 2 ? sl : (form == 1 ? p : t);
 }
 

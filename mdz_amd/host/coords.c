@@ -25,8 +25,18 @@
 
 #include "mdzg_host.h"
 
-const int mdzg_nwords[MDZG_NCLASS_N] = MDZG_NWORDS_INIT;
+static const int nwords[MDZG_NCLASS_N] = MDZG_NWORDS_INIT;
+static const int rn_kid[MDZG_NCLASS_N] = MDZG_RN_KID_INIT;
 const int mdzg_gmp_limbs[MDZG_NGMP] = MDZG_GMP_LIMBS_INIT;
+
+/* words of an RN kernel id, 0 for another */
+int mdzg_kid_words(int kid)
+{
+    for (int i = 0; i < MDZG_NCLASS_N; ++i)
+        if (kid == rn_kid[i] || kid == rn_kid[i] + 1)
+            return nwords[i];
+    return 0;
+}
 
 /* GMP's limb precision of mpf_init2(x, p): __GMPF_BITS_TO_PREC (gmp.h) */
 static long gmp_prec_limbs(long p)
@@ -59,10 +69,10 @@ int mdzg_class_of(int path, long precision, int* nw, int* kclr)
     if (p < 2 || p > MDZG_MAX_PRECISION)
         return -1;
     for (int i = 0; i < MDZG_NCLASS_N; ++i) {
-        if (32L * mdzg_nwords[i] >= p) {
-            *nw = mdzg_nwords[i];
-            *kclr = (int)(32L * mdzg_nwords[i] - p);
-            return 1 + 2 * i + (*kclr == 0 ? 1 : 0);
+        if (32L * nwords[i] >= p) {
+            *nw = nwords[i];
+            *kclr = (int)(32L * nwords[i] - p);
+            return rn_kid[i] + (*kclr == 0 ? 1 : 0);
         }
     }
     return -1;

@@ -76,7 +76,7 @@ int mdzg_rt_submit_image(mdzg_ctx* c, const mdzg_tile* tile, const mdzg_image_re
 /* validation shared by the colouring entry points */
 int mdzg_palette_ok(const mdzg_palette* p);
 
-extern const int mdzg_nwords[MDZG_NCLASS_N];
+int mdzg_kid_words(int kid);   /* words of an RN kernel id, 0 for another */
 extern const int mdzg_gmp_limbs[MDZG_NGMP];
 
 /* A parsed view: image_info fields as MPFR values at max(p, 80) bits; on the

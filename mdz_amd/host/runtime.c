@@ -113,9 +113,8 @@ static int default_chunk(int kid)
 {
     if (kid == 0)
         return 256;
-    if (kid >= 1 && kid < MDZG_KID_GMP0)
-        return mdzg_nwords[(kid - 1) >> 1] <= 2 ? 16 : 8;
-    return 8;
+    const int nw = mdzg_kid_words(kid);
+    return nw >= 1 && nw <= 2 ? 16 : 8;
 }
 
 int mdzg_create(int device, mdzg_ctx** out)

@@ -756,11 +756,9 @@ int mdzg_server_create(mdzg_ctx* ctx, const mdzg_server_cfg* cfg, mdzg_server** 
                 s->occ_slice[k] = 1;
             const int lanes = ctx->ncu * s->occ_slice[k] * 256;
             s->budget_pix[k] = (long long)(s->cfg.occupancy_budget * (double)lanes);
-            int nw = 0;
-            if (k >= MDZG_KID_GMP0)       /* GMP path: limbs of 64 bits */
+            int nw = mdzg_kid_words(k);
+            if (k >= MDZG_KID_GMP0 && k < MDZG_KID_GMP0 + MDZG_NGMP)   /* 64-bit limbs */
                 nw = 2 * mdzg_gmp_limbs[k - MDZG_KID_GMP0];
-            else if (k > 0)
-                nw = mdzg_nwords[(k - 1) >> 1];
             s->slice_iters[k] = s->cfg.slice_iters > 0 ? s->cfg.slice_iters : default_slice_iters(nw);
         }
         if (hipEventCreateWithFlags(&s->ev_fork, hipEventDisableTiming) != hipSuccess) {
