@@ -28,6 +28,7 @@
 #include <stdint.h>
 
 #include "mdzg_dev.h"
+#include "mp_fast.h"
 #include "mp_rn.h"
 
 #pragma clang fp contract(off)
@@ -147,6 +148,16 @@ constexpr uint32_t claim_run()
     return N <= 2 ? 64u : 0u;
 }
 
+/* v + 1 on the lanes set in the lane mask m, v elsewhere: one
+   v_addc_co_u32 with m as the carry-in */
+__device__ __forceinline__ int32_t add_lanes(int32_t v, uint64_t m)
+{
+    int32_t r;
+    uint64_t co;
+    asm("v_addc_co_u32 %0, %1, 0, %2, %3" : "=v"(r), "=s"(co) : "v"(v), "s"(m));
+    return r;
+}
+
 #ifdef MDZG_FP64_KERNELS
 /* ------------------------------------------------------------------ */
 /* FP64                                                                 */
@@ -212,16 +223,6 @@ __global__ __launch_bounds__(256) void k_fp64_tile(const mdzg_dtile* tp)
             break;
     }
     t.out[idx] = count;
-}
-
-/* v + 1 on the lanes set in the lane mask m, v elsewhere: one
-   v_addc_co_u32 with m as the carry-in */
-__device__ __forceinline__ int32_t add_lanes(int32_t v, uint64_t m)
-{
-    int32_t r;
-    uint64_t co;
-    asm("v_addc_co_u32 %0, %1, 0, %2, %3" : "=v"(r), "=s"(co) : "v"(v), "s"(m));
-    return r;
 }
 
 /* One iteration of formula F (a compile-time constant) for every lane of the
@@ -546,6 +547,7 @@ __device__ __forceinline__ void load_mp(mp<N>& v, const uint32_t* p)
     for (int j = 0; j < N; ++j) v.m[j] = p[j];
     v.e = (int32_t)p[N];
     v.s = p[N + 1];
+    clamp_zero<N>(v);
 }
 
 /* minimum waves per SIMD the RN kernels are compiled for: small N keep
@@ -553,7 +555,7 @@ __device__ __forceinline__ void load_mp(mp<N>& v, const uint32_t* p)
 template <int N, bool FULL>
 constexpr int rn_min_waves()
 {
-    return (N >= 32 && !FULL) ? 1 : (N >= 12 ? 2 : 4);
+    return (N >= 32 && !FULL) ? 1 : (N >= 12 ? 2 : (N >= 5 ? 3 : 4));
 }
 
 /* the slice kernel keeps its resume and save paths live inside the
@@ -719,6 +721,31 @@ __device__ __forceinline__ bool rn_step(rn_state<N>& s, int fractal, int32_t wz,
     return escaped<N>(s.wim2, s.wre2, thresh, k);
 }
 
+/* a tile's formula for step_fast */
+__device__ __forceinline__ rn_form form_of(int fractal)
+{
+    rn_form f;
+    f.bs = fractal == F_BURNING_SHIP ? 0u : 1u;
+    f.ce = fractal == F_GENERALIZED_CELTIC ? 0u : 1u;
+    f.va = fractal == F_VARIANT ? 1u : 0u;
+    return f;
+}
+
+/* Up to n iterations (step_fast) of the lanes of live, fewer once none is
+   left; a lane that escapes leaves live, with its count in wz.  Lanes outside
+   live compute on their last values, which nothing reads: no branch of the
+   loop depends on a lane. */
+template <int N, bool FULL>
+__device__ __forceinline__ void rn_run(rn_state<N>& s, const rn_form& f, const rn_prec<FULL>& pr,
+                                       int32_t& wz, lanes& live, int n)
+{
+    for (int it = 0; it < n && live != 0; ++it) {
+        wz = add_lanes(wz, live);
+        live &= ~step_fast<N, FULL>(s.wre, s.wim, s.wre2, s.wim2, s.c.get_re(), s.c.get_im(), f,
+                                    pr, wz, live);
+    }
+}
+
 template <int N, bool FULL>
 __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_tile(const mdzg_dtile* tp)
 {
@@ -735,13 +762,23 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_tile(cons
     const int fractal = t.fractal, kclr = t.kclr;
     const int32_t depth = t.depth;
     uint32_t count = 0;
-    for (int32_t wz = 1;; ++wz) {
-        if (rn_step<N, FULL, true>(s, fractal, wz, kclr)) {
-            count = (uint32_t)wz;
-            break;
+    if constexpr (rn_fast<N>()) {
+        rn_prec<FULL> pr;
+        set_prec(pr, kclr);
+        int32_t wz = 0;
+        const lanes start = scalar_copy(lanes_of(true));
+        lanes live = start;
+        rn_run<N, FULL>(s, form_of(fractal), pr, wz, live, depth);
+        count = ((start & ~live) >> __lane_id()) & 1u ? (uint32_t)wz : 0u;
+    } else {
+        for (int32_t wz = 1;; ++wz) {
+            if (rn_step<N, FULL, true>(s, fractal, wz, kclr)) {
+                count = (uint32_t)wz;
+                break;
+            }
+            if (wz >= depth)
+                break;
         }
-        if (wz >= depth)
-            break;
     }
     t.out[idx] = count;
 }
@@ -846,6 +883,10 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
        frame at 128 bits: +2.5 %).  Not from 24 words: the start-up code changed the register
        allocation of those 256-VGPR kernels, 6 % slower on the 1024-bit band,
        whose launches never fit their lanes. */
+    rn_form fm = { 1u, 1u, 0u };
+    rn_prec<FULL> pr;
+    set_prec(pr, 0);
+    int rem = 0;
     const bool by_lane = N < 24 && total <= (uint64_t)gridDim.x * blockDim.x;
     if (by_lane) {
         run.base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
@@ -869,19 +910,42 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
                 wz = 0;
                 active = true;
                 asm volatile("" ::"v"(fractal), "v"(kclr), "v"(depth), "v"(out));
+                if constexpr (rn_fast<N>()) {
+                    fm = form_of(fractal);
+                    set_prec(pr, kclr);
+                }
             }
+            rem = 0;
             drained = by_lane || __any(need && g >= total);
         }
         if (!__any(active))
             break;
         const int stop = ((++round & 15) == 0) ? read_cancel(cancel) : 0;
-        for (int it = 0; it < chunk; ++it) {
-            if (active) {
-                ++wz;
-                const bool esc = rn_step<N, FULL, true>(s, fractal, wz, kclr);
-                if (esc || wz >= depth) {
-                    put_count(out, esc ? (uint32_t)wz : 0u);
-                    active = false;
+        if constexpr (rn_fast<N>()) {
+            /* no active lane reaches its depth within rem iterations: lanes
+               that finish leave it a bound, a refill (rem = 0) does not */
+            if (rem < chunk)
+                rem = __builtin_amdgcn_readfirstlane(
+                    __ockl_wfred_min_i32(active ? depth - wz : 0x7fffffff));
+            const int n = rem < chunk ? rem : chunk;
+            const lanes start = scalar_copy(__ballot(active));
+            lanes live = start;
+            rn_run<N, FULL>(s, fm, pr, wz, live, n);
+            rem -= n;
+            const bool esc = ((start & ~live) >> __lane_id()) & 1u;
+            if (active && (esc || wz >= depth)) {
+                put_count(out, esc ? (uint32_t)wz : 0u);
+                active = false;
+            }
+        } else {
+            for (int it = 0; it < chunk; ++it) {
+                if (active) {
+                    ++wz;
+                    const bool esc = rn_step<N, FULL, true>(s, fractal, wz, kclr);
+                    if (esc || wz >= depth) {
+                        put_count(out, esc ? (uint32_t)wz : 0u);
+                        active = false;
+                    }
                 }
             }
         }
@@ -915,6 +979,9 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
     __shared__ uint32_t c_lds[c_in_lds<N>() ? 2 * (N + 2) * 256 : 1];
     rn_state<N> s;
     s.c.init(c_lds);
+    rn_form fm = { 1u, 1u, 0u };
+    rn_prec<FULL> pr;
+    set_prec(pr, 0);
     bool drained = false;
     wave_run run = { 0, 0u };
     /* the claim loop runs until the wave holds a pixel or the queue is
@@ -959,13 +1026,46 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
                 depth = tp->depth;
                 left = budget;
                 active = true;
+                if constexpr (rn_fast<N>()) {
+                    fm = form_of(fractal);
+                    set_prec(pr, kclr);
+                }
             }
           }
           drained = __any(need && g >= total) || !__any(lb > 0);
         } while (!__any(active));
         if (!__any(active))
             break;
-        if (active) {
+        if constexpr (rn_fast<N>()) {
+            /* a run that no lane's depth or budget ends: as in k_rn_persist,
+               at most 8 iterations between claims */
+            const int32_t mine = left < lb ? left : lb;
+            const int32_t todo = depth - wz;
+            const int rem = __builtin_amdgcn_readfirstlane(
+                __ockl_wfred_min_i32(active ? (todo < mine ? todo : mine) : 8));
+            const int32_t wz0 = wz;
+            const lanes start = scalar_copy(__ballot(active));
+            lanes live = start;
+            rn_run<N, FULL>(s, fm, pr, wz, live, rem < 8 ? rem : 8);
+            const bool esc = ((start & ~live) >> __lane_id()) & 1u;
+            if (active) {
+                left -= wz - wz0;
+                lb -= wz - wz0;
+                if (esc || wz >= depth) {
+                    put_count(tp->out + local, esc ? (uint32_t)wz : 0u);
+                    atomicSub(tp->remaining, 1u);
+                    active = false;
+                } else if (left == 0 || lb == 0) {
+                    uint32_t* st = tp->state + (size_t)local * 4 * MDZG_VS(N);
+                    store_mp<N>(st, s.wre);
+                    store_mp<N>(st + MDZG_VS(N), s.wim);
+                    store_mp<N>(st + 2 * MDZG_VS(N), s.wre2);
+                    store_mp<N>(st + 3 * MDZG_VS(N), s.wim2);
+                    tp->wzs[local] = wz;
+                    active = false;
+                }
+            }
+        } else if (active) {
             ++wz;
             --left;
             --lb;
