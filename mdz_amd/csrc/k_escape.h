@@ -148,6 +148,21 @@ constexpr uint32_t claim_run()
     return N <= 2 ? 64u : 0u;
 }
 
+/* Orbits that have become periodic.  z_(n+1) is a function of z_n alone (and,
+   for the hybrid formula, of n's parity): the squares that the loop carries
+   are functions of z.  So once z equals, bit for bit, the z of an earlier
+   iteration (of the same parity), none of whose successors escaped, the pixel
+   never escapes and its count is 0, as running to its depth would find.  In
+   p-bit arithmetic an orbit attracted to a cycle lands on one after about p
+   ln 2 / -ln |multiplier| iterations: a hundred or two over most of the set,
+   where views ask for thousands.  A lane keeps one earlier z and compares at
+   intervals (Brent's method): the k-th comparison's z replaces it when k is 1,
+   2, 3, 4, 6, 8, 12, ... */
+__device__ __forceinline__ bool cycle_renew(uint32_t k)
+{
+    return __popc(k) - ((k & (k >> 1)) != 0 ? 1 : 0) == 1;
+}
+
 /* v + 1 on the lanes set in the lane mask m, v elsewhere: one
    v_addc_co_u32 with m as the carry-in */
 __device__ __forceinline__ int32_t add_lanes(int32_t v, uint64_t m)
@@ -202,6 +217,47 @@ __device__ __forceinline__ bool fp64_step(fp64_state& s, int fractal, int32_t wz
     return s.wim2 + s.wre2 > 4.0;
 }
 
+/* Iterations between comparisons of the FP64 loops.  A cycle of length q is
+   seen when the distance to the kept z is a multiple of q: 60 is one for q =
+   1..6, 10, 12, 15, 20 and 30.  The persistent kernel's runs keep one z a
+   lane and replace it on all lanes at once, after 60, 120, 180, 240, 360 ...
+   iterations of the run: four instructions and a vote in about 600.  A lane
+   that starts a pixel forgets its z (a NaN, which no orbit but one of NaNs,
+   never past the escape test either, equals). */
+#ifndef MDZG_CYCLE_FP64
+#define MDZG_CYCLE_FP64 60
+#endif
+
+struct fp64_cycle {
+    uint64_t re, im;   /* the kept z */
+    uint32_t odd;      /* hybrid formula: its iteration's parity */
+};
+
+__device__ __forceinline__ void fp64_forget(fp64_cycle& c)
+{
+    c.re = c.im = ~0ull;
+    c.odd = 0;
+}
+
+/* lanes whose z is the kept one */
+template <int F>
+__device__ __forceinline__ uint64_t fp64_periodic(const fp64_cycle& c, const fp64_state& s,
+                                                  int32_t wz)
+{
+    bool same = (uint64_t)__double_as_longlong(s.wre) == c.re &&
+                (uint64_t)__double_as_longlong(s.wim) == c.im;
+    if (F == F_VARIANT)
+        same = same && ((uint32_t)wz & 1u) == c.odd;
+    return __builtin_amdgcn_ballot_w64(same);
+}
+
+__device__ __forceinline__ void fp64_keep(fp64_cycle& c, const fp64_state& s, int32_t wz)
+{
+    c.re = __double_as_longlong(s.wre);
+    c.im = __double_as_longlong(s.wim);
+    c.odd = (uint32_t)wz & 1u;
+}
+
 __global__ __launch_bounds__(256) void k_fp64_tile(const mdzg_dtile* tp)
 {
     const mdzg_dtile t = *tp;
@@ -213,6 +269,10 @@ __global__ __launch_bounds__(256) void k_fp64_tile(const mdzg_dtile* tp)
     fp64_state s;
     fp64_init(s, t, row, col);
     uint32_t count = 0;
+    fp64_cycle cyc;
+    fp64_forget(cyc);
+    uint32_t k = 0;
+    int until = MDZG_CYCLE_FP64;
     /* the exit test follows the step, so depth == INT32_MAX ends too */
     for (int32_t wz = 1;; ++wz) {
         if (fp64_step(s, t.fractal, wz)) {
@@ -221,6 +281,13 @@ __global__ __launch_bounds__(256) void k_fp64_tile(const mdzg_dtile* tp)
         }
         if (wz >= t.depth)
             break;
+        if (--until == 0) {
+            until = MDZG_CYCLE_FP64;
+            if ((fp64_periodic<F_VARIANT>(cyc, s, wz) >> __lane_id()) & 1u)
+                break;
+            if (cycle_renew(++k))
+                fp64_keep(cyc, s, wz);
+        }
     }
     t.out[idx] = count;
 }
@@ -250,24 +317,40 @@ __device__ __forceinline__ void fp64_iter(fp64_state& s, int32_t& wz, uint64_t& 
 }
 
 /* Up to n iterations of formula F, fewer once no lane is left iterating;
-   escm gets the lanes that escaped.  Without DEPTH the caller has checked
-   that no live lane reaches its depth within n iterations. */
+   escm gets the lanes that escaped; periodic lanes leave live, too.  Without
+   DEPTH the caller has checked that no live lane reaches its depth within n
+   iterations. */
 template <int F, bool DEPTH>
 __device__ __forceinline__ void fp64_run(fp64_state& s, int32_t& wz, uint64_t& live,
-                                         uint64_t& escm, int32_t depth, int n)
+                                         uint64_t& escm, fp64_cycle& cyc, int32_t depth, int n)
 {
     const uint64_t start = live;
-    int it = 0;
-    for (; it + 4 <= n && live != 0; it += 4) {
-        fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
-        fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
-        fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
-        fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
+    uint64_t per = 0;
+    uint32_t k = 0;
+    for (int it = 0; it < n && live != 0;) {
+        const int stop = n - it > MDZG_CYCLE_FP64 ? it + MDZG_CYCLE_FP64 : n;
+        /* an exit test and the loop's own scalar work cost a wave about 80
+           cycles, an iteration 54: a test every 4 iterations while pixels are
+           new (most escape soon), then every 12 */
+        const int first = it == 0 ? (stop < 12 ? stop : 12) : it;
+        for (; it + 4 <= first && live != 0; it += 4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
+        }
+        for (; it + 12 <= stop && live != 0; it += 12) {
+#pragma unroll
+            for (int j = 0; j < 12; ++j) fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
+        }
+        for (; it < stop && live != 0; ++it)
+            fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
+        const uint64_t p = fp64_periodic<F>(cyc, s, wz) & live;
+        per |= p;
+        live &= ~p;
+        if (cycle_renew(++k))
+            fp64_keep(cyc, s, wz);
     }
-    for (; it < n && live != 0; ++it)
-        fp64_iter<F, DEPTH>(s, wz, live, escm, depth);
     if (!DEPTH)
-        escm = start & ~live;
+        escm = start & ~live & ~per;
 }
 
 /* The latency form of an iteration, for launches whose pixels all fit the
@@ -292,49 +375,60 @@ __device__ __forceinline__ void fp64_iter_v(fp64_state& s, int32_t& wz, int32_t&
     }
 }
 
-/* fp64_run in the latency form: the wave tests for an exit every 4
-   iterations, as fp64_run does */
+/* fp64_run in the latency form: the wave tests for an exit every 12
+   iterations and compares every 240 (such a launch lasts as long as its
+   slowest pixel, seldom a periodic one) */
+#define MDZG_CYCLE_FP64_LAT 240
 template <int F, bool DEPTH>
 __device__ __forceinline__ void fp64_run_v(fp64_state& s, int32_t& wz, uint64_t& live,
-                                           uint64_t& escm, int32_t depth, int n)
+                                           uint64_t& escm, fp64_cycle& cyc, int32_t depth, int n)
 {
     const uint64_t start = live;
+    uint64_t per = 0;
+    uint32_t k = 0;
     int32_t lv = (int32_t)((live >> __lane_id()) & 1u), ev = 0;
-    int it = 0;
-    for (; it + 4 <= n && __builtin_amdgcn_ballot_w64(lv != 0) != 0; it += 4) {
-        fp64_iter_v<F, DEPTH>(s, wz, lv, ev, depth);
-        fp64_iter_v<F, DEPTH>(s, wz, lv, ev, depth);
-        fp64_iter_v<F, DEPTH>(s, wz, lv, ev, depth);
-        fp64_iter_v<F, DEPTH>(s, wz, lv, ev, depth);
+    for (int it = 0; it < n && __builtin_amdgcn_ballot_w64(lv != 0) != 0;) {
+        const int stop = n - it > MDZG_CYCLE_FP64_LAT ? it + MDZG_CYCLE_FP64_LAT : n;
+        for (; it + 12 <= stop && __builtin_amdgcn_ballot_w64(lv != 0) != 0; it += 12) {
+#pragma unroll
+            for (int j = 0; j < 12; ++j) fp64_iter_v<F, DEPTH>(s, wz, lv, ev, depth);
+        }
+        for (; it < stop && __builtin_amdgcn_ballot_w64(lv != 0) != 0; ++it)
+            fp64_iter_v<F, DEPTH>(s, wz, lv, ev, depth);
+        const uint64_t p = fp64_periodic<F>(cyc, s, wz) & __builtin_amdgcn_ballot_w64(lv != 0);
+        if (p != 0) {
+            per |= p;
+            lv = (p >> __lane_id()) & 1u ? 0 : lv;
+        }
+        if (cycle_renew(++k))
+            fp64_keep(cyc, s, wz);
     }
-    for (; it < n && __builtin_amdgcn_ballot_w64(lv != 0) != 0; ++it)
-        fp64_iter_v<F, DEPTH>(s, wz, lv, ev, depth);
     live = __builtin_amdgcn_ballot_w64(lv != 0);
-    escm = DEPTH ? (escm | __builtin_amdgcn_ballot_w64(ev != 0)) : (start & ~live);
+    escm = DEPTH ? (escm | __builtin_amdgcn_ballot_w64(ev != 0)) : (start & ~live & ~per);
 }
 
 template <bool DEPTH, bool LAT>
 __device__ __forceinline__ void fp64_run_formula(int f, fp64_state& s, int32_t& wz, uint64_t& live,
-                                                 uint64_t& escm, int32_t depth, int n)
+                                                 uint64_t& escm, fp64_cycle& cyc, int32_t depth, int n)
 {
     if (LAT) {
         switch (f) {
-        case F_MANDELBROT: fp64_run_v<F_MANDELBROT, DEPTH>(s, wz, live, escm, depth, n); break;
-        case F_BURNING_SHIP: fp64_run_v<F_BURNING_SHIP, DEPTH>(s, wz, live, escm, depth, n); break;
+        case F_MANDELBROT: fp64_run_v<F_MANDELBROT, DEPTH>(s, wz, live, escm, cyc, depth, n); break;
+        case F_BURNING_SHIP: fp64_run_v<F_BURNING_SHIP, DEPTH>(s, wz, live, escm, cyc, depth, n); break;
         case F_GENERALIZED_CELTIC:
-            fp64_run_v<F_GENERALIZED_CELTIC, DEPTH>(s, wz, live, escm, depth, n);
+            fp64_run_v<F_GENERALIZED_CELTIC, DEPTH>(s, wz, live, escm, cyc, depth, n);
             break;
-        default: fp64_run_v<F_VARIANT, DEPTH>(s, wz, live, escm, depth, n); break;
+        default: fp64_run_v<F_VARIANT, DEPTH>(s, wz, live, escm, cyc, depth, n); break;
         }
         return;
     }
     switch (f) {
-    case F_MANDELBROT: fp64_run<F_MANDELBROT, DEPTH>(s, wz, live, escm, depth, n); break;
-    case F_BURNING_SHIP: fp64_run<F_BURNING_SHIP, DEPTH>(s, wz, live, escm, depth, n); break;
+    case F_MANDELBROT: fp64_run<F_MANDELBROT, DEPTH>(s, wz, live, escm, cyc, depth, n); break;
+    case F_BURNING_SHIP: fp64_run<F_BURNING_SHIP, DEPTH>(s, wz, live, escm, cyc, depth, n); break;
     case F_GENERALIZED_CELTIC:
-        fp64_run<F_GENERALIZED_CELTIC, DEPTH>(s, wz, live, escm, depth, n);
+        fp64_run<F_GENERALIZED_CELTIC, DEPTH>(s, wz, live, escm, cyc, depth, n);
         break;
-    default: fp64_run<F_VARIANT, DEPTH>(s, wz, live, escm, depth, n); break;
+    default: fp64_run<F_VARIANT, DEPTH>(s, wz, live, escm, cyc, depth, n); break;
     }
 }
 
@@ -345,14 +439,15 @@ __device__ __forceinline__ void fp64_run_formula(int f, fp64_state& s, int32_t& 
    took them out), and the rest of the run has the test. */
 template <bool LAT>
 __device__ __forceinline__ void fp64_chunk(int f0, fp64_state& s, int32_t& wz, uint64_t& live,
-                                           uint64_t& escm, int32_t depth, int chunk, int rem)
+                                           uint64_t& escm, fp64_cycle& cyc, int32_t depth, int chunk,
+                                           int rem)
 {
     if (rem >= chunk) {
-        fp64_run_formula<false, LAT>(f0, s, wz, live, escm, depth, chunk);
+        fp64_run_formula<false, LAT>(f0, s, wz, live, escm, cyc, depth, chunk);
     } else {
-        fp64_run_formula<false, LAT>(f0, s, wz, live, escm, depth, rem);
+        fp64_run_formula<false, LAT>(f0, s, wz, live, escm, cyc, depth, rem);
         live &= ~__builtin_amdgcn_ballot_w64(wz >= depth);
-        fp64_run_formula<true, LAT>(f0, s, wz, live, escm, depth, chunk - rem);
+        fp64_run_formula<true, LAT>(f0, s, wz, live, escm, cyc, depth, chunk - rem);
     }
 }
 
@@ -368,6 +463,8 @@ __global__ __launch_bounds__(256) void k_fp64_persist(const mdzg_dtile* tiles, i
     uint32_t* out = nullptr;
     fp64_state s;
     s.wre = s.wim = s.wre2 = s.wim2 = s.cre = s.cim = 0.0;
+    fp64_cycle cyc;
+    fp64_forget(cyc);
     bool drained = false;
     wave_run run = { 0, 0u };
     const uint32_t run_len = share_run(total);
@@ -390,6 +487,7 @@ __global__ __launch_bounds__(256) void k_fp64_persist(const mdzg_dtile* tiles, i
                 depth = t.depth;
                 out = t.out + local;
                 wz = 0;
+                fp64_forget(cyc);
                 active = true;
                 /* the tile's fields are waited for here, on the refill path:
                    a wait where the paths join would also wait, every round,
@@ -428,11 +526,11 @@ __global__ __launch_bounds__(256) void k_fp64_persist(const mdzg_dtile* tiles, i
                iterations update it with scalar instructions) */
             uint64_t live = scalar_copy(am), escm = 0;
             if (by_lane)
-                fp64_chunk<true>(f0, s, wz, live, escm, depth, chunk, rem);
+                fp64_chunk<true>(f0, s, wz, live, escm, cyc, depth, chunk, rem);
             else
-                fp64_chunk<false>(f0, s, wz, live, escm, depth, chunk, rem);
+                fp64_chunk<false>(f0, s, wz, live, escm, cyc, depth, chunk, rem);
             const bool esc = (escm >> __lane_id()) & 1u;
-            if (active && (esc || wz >= depth)) {
+            if (active && (!((live >> __lane_id()) & 1u) || wz >= depth)) {
                 put_count(out, esc ? (uint32_t)wz : 0u);
                 active = false;
             }
@@ -476,6 +574,8 @@ __global__ __launch_bounds__(256) void k_fp64_slice(const mdzg_dtile* tiles, int
     const mdzg_dtile* tp = tiles;
     fp64_state s;
     s.wre = s.wim = s.wre2 = s.wim2 = s.cre = s.cim = 0.0;
+    fp64_cycle cyc;
+    fp64_forget(cyc);
     bool drained = false;
     wave_run run = { 0, 0u };
     for (;;) {
@@ -501,6 +601,7 @@ __global__ __launch_bounds__(256) void k_fp64_slice(const mdzg_dtile* tiles, int
                 fractal = tp->fractal;
                 depth = tp->depth;
                 left = budget;
+                fp64_forget(cyc);
                 active = true;
             }
           }
@@ -511,25 +612,47 @@ __global__ __launch_bounds__(256) void k_fp64_slice(const mdzg_dtile* tiles, int
                 break;
             continue;
         }
-        for (int it = 0; it < 32; ++it) {
+        /* a wave of one formula (the usual case) runs without branches up to
+           the first depth or budget of its lanes, at most two comparisons'
+           distance (a longer run would leave lanes idle that could claim) */
+        const uint64_t am = __ballot(active);
+        const int f0 =
+            __builtin_amdgcn_readfirstlane(__shfl(fractal, __ffsll((long long)am) - 1));
+        bool esc = false, over = false;
+        if (__all(!active || fractal == f0)) {
+            const int32_t mine = left < lb ? left : lb;
+            const int32_t todo = depth - wz;
+            const int n = __builtin_amdgcn_readfirstlane(__ockl_wfred_min_i32(
+                active ? (todo < mine ? todo : mine) : 2 * MDZG_CYCLE_FP64));
+            const int32_t wz0 = wz;
+            uint64_t live = scalar_copy(am), escm = 0;
+            fp64_run_formula<false, false>(f0, s, wz, live, escm, cyc, depth,
+                                           n < 2 * MDZG_CYCLE_FP64 ? n : 2 * MDZG_CYCLE_FP64);
             if (active) {
-                ++wz;
-                --left;
-                --lb;
-                const bool esc = fp64_step(s, fractal, wz);
-                if (esc || wz >= depth) {
-                    put_count(tp->out + local, esc ? (uint32_t)wz : 0u);
-                    atomicSub(tp->remaining, 1u);
-                    active = false;
-                } else if (left == 0 || lb == 0) {
-                    double* st = (double*)tp->state + 4 * (size_t)local;
-                    st[0] = s.wre;
-                    st[1] = s.wim;
-                    st[2] = s.wre2;
-                    st[3] = s.wim2;
-                    tp->wzs[local] = wz;
-                    active = false;
-                }
+                left -= wz - wz0;
+                lb -= wz - wz0;
+                esc = (escm >> __lane_id()) & 1u;
+                over = !((live >> __lane_id()) & 1u);
+            }
+        } else if (active) {
+            ++wz;
+            --left;
+            --lb;
+            esc = fp64_step(s, fractal, wz);
+        }
+        if (active) {
+            if (esc || over || wz >= depth) {
+                put_count(tp->out + local, esc ? (uint32_t)wz : 0u);
+                atomicSub(tp->remaining, 1u);
+                active = false;
+            } else if (left == 0 || lb == 0) {
+                double* st = (double*)tp->state + 4 * (size_t)local;
+                st[0] = s.wre;
+                st[1] = s.wim;
+                st[2] = s.wre2;
+                st[3] = s.wim2;
+                tp->wzs[local] = wz;
+                active = false;
             }
         }
     }
@@ -721,6 +844,50 @@ __device__ __forceinline__ bool rn_step(rn_state<N>& s, int fractal, int32_t wz,
     return escaped<N>(s.wim2, s.wre2, thresh, k);
 }
 
+/* Iterations between comparisons of the RN loops of up to 8 words (about 25
+   instructions in 32 iterations of 200 to 530).  The kept z lies in the
+   block's LDS, word w of lane t at [w][t]: both significands, then the
+   exponents with their signs.  The wider loops make none: views that need
+   them lie too deep for p / -log2 |multiplier| iterations to be few. */
+#define MDZG_CYCLE_RN 32
+
+template <int N>
+constexpr int cycle_words()
+{
+    return rn_fast<N>() ? 2 * N + 2 : 0;
+}
+
+/* true on the lanes of `on` whose orbit is periodic; k counts a lane's
+   comparisons */
+template <int N>
+__device__ __forceinline__ bool rn_periodic(uint32_t* kept, uint32_t& k, const rn_state<N>& s,
+                                            uint32_t hybrid, int32_t wz, bool on)
+{
+    uint32_t* z = kept + threadIdx.x;
+    on = on && !((uint32_t)wz & hybrid);
+    /* the lowest words first: they differ on nearly every orbit */
+    bool hit = on && k != 0 && z[0] == s.wre.m[0] && z[N * 256] == s.wim.m[0];
+    if (wave_any(hit)) {
+        uint32_t d = (z[2 * N * 256] ^ (((uint32_t)s.wre.e << 1) | s.wre.s)) |
+                     (z[(2 * N + 1) * 256] ^ (((uint32_t)s.wim.e << 1) | s.wim.s));
+#pragma unroll
+        for (int j = 1; j < N; ++j)
+            d |= (z[j * 256] ^ s.wre.m[j]) | (z[(N + j) * 256] ^ s.wim.m[j]);
+        hit = hit && d == 0;
+    }
+    k += on ? 1u : 0u;
+    if (on && cycle_renew(k)) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            z[j * 256] = s.wre.m[j];
+            z[(N + j) * 256] = s.wim.m[j];
+        }
+        z[2 * N * 256] = ((uint32_t)s.wre.e << 1) | s.wre.s;
+        z[(2 * N + 1) * 256] = ((uint32_t)s.wim.e << 1) | s.wim.s;
+    }
+    return hit;
+}
+
 /* a tile's formula for step_fast */
 __device__ __forceinline__ rn_form form_of(int fractal)
 {
@@ -756,6 +923,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_tile(cons
         return;
     const int row = (int)(idx / (uint32_t)t.ncols), col = (int)(idx % (uint32_t)t.ncols);
     __shared__ uint32_t c_lds[c_in_lds<N>() ? 2 * (N + 2) * 256 : 1];
+    __shared__ uint32_t kept[cycle_words<N>() * 256 + 1];
     rn_state<N> s;
     s.c.init(c_lds);
     rn_init<N, FULL>(s, t, row, col);
@@ -765,11 +933,20 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_tile(cons
     if constexpr (rn_fast<N>()) {
         rn_prec<FULL> pr;
         set_prec(pr, kclr);
+        const rn_form fm = form_of(fractal);
         int32_t wz = 0;
+        uint32_t seen = 0;
         const lanes start = scalar_copy(lanes_of(true));
-        lanes live = start;
-        rn_run<N, FULL>(s, form_of(fractal), pr, wz, live, depth);
-        count = ((start & ~live) >> __lane_id()) & 1u ? (uint32_t)wz : 0u;
+        lanes live = start, esc = 0;
+        for (int32_t done = 0; done < depth && live != 0;) {
+            const int32_t n = depth - done < MDZG_CYCLE_RN ? depth - done : MDZG_CYCLE_RN;
+            const lanes before = live;
+            rn_run<N, FULL>(s, fm, pr, wz, live, n);
+            esc |= before & ~live;
+            done += n;
+            live &= ~lanes_of(rn_periodic<N>(kept, seen, s, fm.va, wz, (live >> __lane_id()) & 1u));
+        }
+        count = (esc >> __lane_id()) & 1u ? (uint32_t)wz : 0u;
     } else {
         for (int32_t wz = 1;; ++wz) {
             if (rn_step<N, FULL, true>(s, fractal, wz, kclr)) {
@@ -886,7 +1063,9 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
     rn_form fm = { 1u, 1u, 0u };
     rn_prec<FULL> pr;
     set_prec(pr, 0);
-    int rem = 0;
+    int rem = 0, since = 0;
+    uint32_t seen = 0;
+    __shared__ uint32_t kept[cycle_words<N>() * 256 + 1];
     const bool by_lane = N < 24 && total <= (uint64_t)gridDim.x * blockDim.x;
     if (by_lane) {
         run.base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
@@ -913,6 +1092,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
                 if constexpr (rn_fast<N>()) {
                     fm = form_of(fractal);
                     set_prec(pr, kclr);
+                    seen = 0;
                 }
             }
             rem = 0;
@@ -933,7 +1113,13 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
             rn_run<N, FULL>(s, fm, pr, wz, live, n);
             rem -= n;
             const bool esc = ((start & ~live) >> __lane_id()) & 1u;
-            if (active && (esc || wz >= depth)) {
+            bool over = wz >= depth;
+            since += n;
+            if (since >= MDZG_CYCLE_RN) {
+                since = 0;
+                over |= rn_periodic<N>(kept, seen, s, fm.va, wz, active && !esc);
+            }
+            if (active && (esc || over)) {
                 put_count(out, esc ? (uint32_t)wz : 0u);
                 active = false;
             }
@@ -982,6 +1168,9 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
     rn_form fm = { 1u, 1u, 0u };
     rn_prec<FULL> pr;
     set_prec(pr, 0);
+    int since = 0;
+    uint32_t seen = 0;
+    __shared__ uint32_t kept[cycle_words<N>() * 256 + 1];
     bool drained = false;
     wave_run run = { 0, 0u };
     /* the claim loop runs until the wave holds a pixel or the queue is
@@ -1029,6 +1218,7 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
                 if constexpr (rn_fast<N>()) {
                     fm = form_of(fractal);
                     set_prec(pr, kclr);
+                    seen = 0;
                 }
             }
           }
@@ -1048,10 +1238,16 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
             lanes live = start;
             rn_run<N, FULL>(s, fm, pr, wz, live, rem < 8 ? rem : 8);
             const bool esc = ((start & ~live) >> __lane_id()) & 1u;
+            bool over = wz >= depth;
+            since += rem < 8 ? rem : 8;
+            if (since >= MDZG_CYCLE_RN) {
+                since = 0;
+                over |= rn_periodic<N>(kept, seen, s, fm.va, wz, active && !esc);
+            }
             if (active) {
                 left -= wz - wz0;
                 lb -= wz - wz0;
-                if (esc || wz >= depth) {
+                if (esc || over) {
                     put_count(tp->out + local, esc ? (uint32_t)wz : 0u);
                     atomicSub(tp->remaining, 1u);
                     active = false;
