@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#define MDZG_CUTS_BOUNDED
 #include "mdzg_dev.h"
 #include "mp_fast.h"
 #include "mp_rn.h"
@@ -674,21 +675,22 @@ __device__ __forceinline__ void load_mp(mp<N>& v, const uint32_t* p)
 }
 
 /* minimum waves per SIMD the RN kernels are compiled for: small N keep
-   several waves resident, large N get the register file to themselves */
+   several waves resident, large N share the register file by two (the ragged
+   32-word class, too, since its rounding masks only the cut's words: 1.35
+   times the pixel rate of one wave) */
 template <int N, bool FULL>
 constexpr int rn_min_waves()
 {
-    return (N >= 32 && !FULL) ? 1 : (N >= 12 ? 2 : (N >= 5 ? 3 : 4));
+    return N >= 12 ? 2 : (N >= 5 ? 3 : 4);
 }
 
 /* the slice kernel keeps its resume and save paths live inside the
    iteration loop, so it gets a larger share of the register file than the
-   other kernels from 8 words up: two waves per SIMD (one for the ragged
-   32-word class, as the other kernels) */
+   other kernels from 8 words up: two waves per SIMD */
 template <int N, bool FULL>
 constexpr int rn_min_waves_slice()
 {
-    return (N >= 32 && !FULL) ? 1 : (N >= 8 ? 2 : rn_min_waves<N, FULL>());
+    return N >= 8 ? 2 : rn_min_waves<N, FULL>();
 }
 
 /* c per lane: registers for small N; for N >= 24 the block's LDS (word w of

@@ -86,16 +86,6 @@ MP_HD lanes join(lanes a, lanes b)
 #endif
 }
 
-/* x, unknown to the optimiser: an exponent read again on a path that is
-   hardly ever taken, so that the path does not keep the loop's own sums of
-   exponents alive (which costs the loop a copy each) */
-MP_HD int32_t again(int32_t x)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm("" : "+v"(x));
-#endif
-    return x;
-}
 template <int N>
 MP_HD mp<N> again(const mp<N>& v)
 {

@@ -247,50 +247,88 @@ MP_HD bool wave_all(bool c)
 #endif
 }
 
-/* kclr = 32N - p in [1, 32N-1]: clear the low kclr bits of R, round at bit kclr */
+/* x, unknown to the optimiser: an exponent read again on a path that is
+   hardly ever taken, so that the path does not keep the loop's own sums of
+   exponents alive (which costs the loop a copy each), or a precision, so that
+   the masks made of it are not moved out of the loop */
+MP_HD int32_t again(int32_t x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(x));
+#endif
+    return x;
+}
+
+/* words that hold the cut of the precisions that run at N words (the word
+   counts step by 1 up to 8, by 2 up to 16, by 4 up to 32) */
+#ifdef MDZG_CUTS_BOUNDED   /* the kernels: every kclr is at most 32 cut_words<N>() */
+static constexpr bool CUTS_BOUNDED = true;
+#else
+static constexpr bool CUTS_BOUNDED = false;
+#endif
+template <int N>
+constexpr int cut_words() { return N <= 8 ? 1 : (N <= 16 ? 2 : 4); }
+
+/* kclr = 32N - p in [1, 32N-1]: clear the low kclr bits of R, round at bit
+   kclr.  In the kernels the round bit lies in one of the cut_words<N>()
+   lowest words, and only those are masked: with masks on every word a
+   rounding took more instructions than the addition it followed, and the
+   masks, moved out of the loop, spilled registers in the ragged kernels from
+   10 words up (again() keeps them in).  512x512 frames at 400, 800, 900 and
+   1000 bits: 15.5 -> 9.9, 89.7 -> 45.6, 101 -> 59.6, 80 -> 59.4 ms. */
 template <int N>
 MP_HD void round_masked(uint32_t* R, uint32_t G, uint32_t S, int32_t& e, int kclr)
 {
-    if (N == 1 || wave_all(kclr < 32)) {
-        /* the rounding position lies in the lowest word (p = 80, 100, 176,
-           184, ...; always for N = 1, where p >= 2): only word 0 is masked,
-           the increment ripples upward as in add_ulp */
-        const uint32_t rm = 1u << (kclr - 1);            /* round bit */
-        const uint32_t rbit = R[0] & rm;
-        const uint32_t st = G | S | (R[0] & (rm - 1u));  /* sticky    */
-        const uint32_t lsb = R[0] & (rm << 1);           /* kept lsb  */
-        R[0] &= ~((rm << 1) - 1u);
-        const uint32_t inc = (uint32_t)(rbit != 0) & (uint32_t)((st != 0) | (lsb != 0));
-        add_ulp<N>(R, e, inc << kclr);
+    if (N == 1 || (CUTS_BOUNDED && cut_words<N>() == 1) || wave_all(kclr <= 32)) {
+        /* word 0 (p = 80, 100, 176, 184, ...): {R[0] below the kept part, G,
+           S} + half - 1 + the kept part's last bit carries into the kept
+           part exactly where nearest even rounds up */
+        const uint32_t b = (uint32_t)(kclr - 1) & 31u;
+        const uint32_t half = 1u << b;
+        uint32_t c;
+        const uint32_t lsb = (funnel_r(N > 1 ? R[N > 1 ? 1 : 0] : 0u, R[0], b) >> 1) & 1u;
+        R[0] = add_cc(R[0], half - 1u, (G | S | lsb) != 0 ? 1u : 0u, c) & (0u - (half << 1));
+        if (N > 1)
+            R[N > 1 ? 1 : 0] = add_cc(R[N > 1 ? 1 : 0], 0u, c, c);
+        if (__builtin_expect(wave_any(c != 0), 0)) {
+#pragma unroll
+            for (int j = 2; j < N; ++j) R[j] = add_cc(R[j], 0u, c, c);
+            if (c) {
+                R[N - 1] = 0x80000000u;
+                e += 1;
+            }
+        }
         return;
     }
-    const int wi = kclr >> 5, bi = kclr & 31;            /* lsb of the kept part */
-    const int rr = kclr - 1, rw = rr >> 5, rb = rr & 31; /* round bit            */
-    uint32_t rbit = 0, st = G | S, lsb = 0;
+    constexpr int W = CUTS_BOUNDED && cut_words<N>() < N ? cut_words<N>() : N;
+    kclr = again(kclr);
+    const int rw = (kclr - 1) >> 5;                      /* word of the round bit */
+    const uint32_t b = (uint32_t)(kclr - 1) & 31u;
+    const uint32_t half = 1u << b;
+    const uint32_t keep = 0u - (half << 1);
+    uint32_t z = G | S;
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const uint32_t keep = (j > wi) ? 0xffffffffu : (j == wi ? (0xffffffffu << bi) : 0u);
-        const uint32_t rm = (j == rw) ? (1u << rb) : 0u;
-        const uint32_t sm = (j < rw) ? 0xffffffffu : (j == rw ? ((1u << rb) - 1u) : 0u);
-        const uint32_t lm = (j == wi) ? (1u << bi) : 0u;
-        rbit |= R[j] & rm;
-        st |= R[j] & sm;
-        lsb |= R[j] & lm;
-        R[j] &= keep;
+    for (int j = 0; j < W; ++j) {
+        const uint32_t l = (funnel_r(j + 1 < N ? R[j + 1 < N ? j + 1 : 0] : 0u, R[j], b) >> 1) & 1u;
+        z |= j < rw ? R[j] : (j == rw ? l : 0u);
     }
-    const uint32_t inc = (uint32_t)(rbit != 0) & (uint32_t)((st != 0) | (lsb != 0));
-    /* add inc << kclr: word wi gets inc << bi, carries ripple upward
-       (words below wi are zero and receive nothing) */
     uint32_t c = 0;
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const uint32_t add = (j == wi) ? (inc << bi) : 0u;
-        const uint32_t cin = (j > wi) ? c : 0u;
-        R[j] = add_cc(R[j], add, cin, c);
+    for (int j = 0; j < W; ++j) {
+        const bool at = j == rw;
+        const uint32_t t = add_cc(R[j], at ? half - 1u : 0u, at ? (z != 0 ? 1u : 0u) : c, c);
+        R[j] = j < rw ? 0u : (at ? t & keep : t);
+        c = j < rw ? 0u : c;
     }
-    if (c) {
-        R[N - 1] = 0x80000000u;
-        e += 1;
+    if (W < N)
+        R[W < N ? W : 0] = add_cc(R[W < N ? W : 0], 0u, c, c);
+    if (wave_any(c != 0)) {
+#pragma unroll
+        for (int j = W + 1; j < N; ++j) R[j] = add_cc(R[j], 0u, c, c);
+        if (c) {
+            R[N - 1] = 0x80000000u;
+            e += 1;
+        }
     }
 }
 
