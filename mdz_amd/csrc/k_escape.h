@@ -693,13 +693,13 @@ constexpr int rn_min_waves_slice()
     return N >= 8 ? 2 : rn_min_waves<N, FULL>();
 }
 
-/* c per lane: registers for small N; for N >= 24 the block's LDS (word w of
+/* c per lane: registers for small N; for N >= 20 the block's LDS (word w of
    lane t at [w][t], conflict-free), so the register file holds z and z^2 only
    and two waves fit per SIMD */
 template <int N>
 constexpr bool c_in_lds()
 {
-    return N >= 24;
+    return N >= 20;
 }
 
 template <int N, bool LDS>
@@ -750,9 +750,59 @@ struct c_src<N, true> {
 template <int N>
 struct rn_state {
     mp<N> wre, wim, wre2, wim2;
+    limb_value<limb_product<N>() ? N : 1> lre, lim;   /* wide N: z in limbs (rn_z) */
     c_src<N, c_in_lds<N>()> c;
     bool lazy;   /* wim2 holds only a bound on its exponent (rn_step, LAZY) */
 };
+
+/* From 20 words up z is kept in the limbs that its products read, made once
+   an iteration, and in words only where it is stored: rn_z after the words
+   were set, rn_words before they are read. */
+template <int N>
+__device__ __forceinline__ void rn_z(rn_state<N>& s)
+{
+    if constexpr (limb_product<N>()) {
+        to_limbs<N>(s.lre, s.wre);
+        to_limbs<N>(s.lim, s.wim);
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void rn_words(rn_state<N>& s)
+{
+    if constexpr (limb_product<N>()) {
+        from_limbs<N>(s.wre, s.lre);
+        from_limbs<N>(s.wim, s.lim);
+    }
+}
+
+/* r = re^2, im^2 or re * im of z */
+template <int N>
+__device__ __forceinline__ void sqr_re(mp<N>& r, const rn_state<N>& s, int k)
+{
+    if constexpr (limb_product<N>())
+        mul_limbs<N, true>(r, s.lre, s.lre, k);
+    else
+        mul_rn<N, true>(r, s.wre, s.wre, k);
+}
+
+template <int N>
+__device__ __forceinline__ void sqr_im(mp<N>& r, const rn_state<N>& s, int k)
+{
+    if constexpr (limb_product<N>())
+        mul_limbs<N, true>(r, s.lim, s.lim, k);
+    else
+        mul_rn<N, true>(r, s.wim, s.wim, k);
+}
+
+template <int N>
+__device__ __forceinline__ void mul_re_im(mp<N>& r, const rn_state<N>& s, int k)
+{
+    if constexpr (limb_product<N>())
+        mul_limbs<N, false>(r, s.lre, s.lim, k);
+    else
+        mul_rn<N, false>(r, s.wre, s.wim, k);
+}
 
 template <int N, bool FULL>
 __device__ __forceinline__ void rn_init(rn_state<N>& s, const mdzg_dtile& t, int row, int col)
@@ -760,8 +810,9 @@ __device__ __forceinline__ void rn_init(rn_state<N>& s, const mdzg_dtile& t, int
     const int k = FULL ? 0 : t.kclr;
     load_mp<N>(s.wre, t.xs + (size_t)col * MDZG_VS(N));
     load_mp<N>(s.wim, t.ys + (size_t)row * MDZG_VS(N));
-    mul_rn<N, true>(s.wre2, s.wre, s.wre, k);      /* src/fractal.c:188 */
-    mul_rn<N, true>(s.wim2, s.wim, s.wim, k);      /* src/fractal.c:171 */
+    rn_z<N>(s);
+    sqr_re<N>(s.wre2, s, k);                       /* src/fractal.c:188 */
+    sqr_im<N>(s.wim2, s, k);                       /* src/fractal.c:171 */
     s.lazy = false;
     if (t.family == 1) {
         mp<N> jr, ji;
@@ -806,21 +857,24 @@ __device__ __forceinline__ bool rn_step(rn_state<N>& s, int fractal, int32_t wz,
         if (__builtin_expect(wave_any(s.lazy) &&
                                  !wave_all((int64_t)s.wre2.e - s.wim2.e >= GAP), 0)) {
             mp<N> sq;
-            mul_rn<N, true>(sq, s.wim, s.wim, k);
+            sqr_im<N>(sq, s, k);
             if (s.lazy)
                 s.wim2 = sq;
             s.lazy = false;
         }
     }
-    mp<N> t;
-    mul_rn<N, false>(t, s.wre, s.wim, k);                    /* t1 = wre*wim     */
+    /* the squares' difference before the product: where a product's limbs
+       fill the registers, the squares no longer do */
+    mp<N> t, u;
+    add_rn<N, SUB_NONNEG, FULL>(u, s.wre2, s.wim2, 1u, k);   /* t1 = wre2 - wim2 */
+    mul_re_im<N>(t, s, k);                                   /* t1 = wre*wim     */
     t.s = (fractal == F_BURNING_SHIP) ? 0u : t.s;            /* BS: |t1|         */
     twice<N>(t);                                             /* t1 *= 2          */
     add_rn<N>(s.wim, t, s.c.get_im(), 0u, k);                /* wim = t1 + c_im  */
-    add_rn<N, SUB_NONNEG, FULL>(t, s.wre2, s.wim2, 1u, k);   /* t1 = wre2 - wim2 */
     const bool ab = fractal == F_GENERALIZED_CELTIC || (fractal == F_VARIANT && (wz & 1));
-    t.s = ab ? 0u : t.s;                                     /* Celtic: |t1|     */
-    add_rn<N>(s.wre, t, s.c.get_re(), 0u, k);                /* wre = t1 + c_re  */
+    u.s = ab ? 0u : u.s;                                     /* Celtic: |t1|     */
+    add_rn<N>(s.wre, u, s.c.get_re(), 0u, k);                /* wre = t1 + c_re  */
+    rn_z<N>(s);
     if constexpr (LZ) {
         /* e(wim^2) <= 2 e(wim) + 1 and e(wre^2) >= 2 e(wre) - 1 */
         const int64_t eb = 2 * (int64_t)s.wim.e + 1;
@@ -834,13 +888,13 @@ __device__ __forceinline__ bool rn_step(rn_state<N>& s, int fractal, int32_t wz,
             s.wim2.s = 0;
             s.lazy = true;
         } else {
-            mul_rn<N, true>(s.wim2, s.wim, s.wim, k);        /* wim2 = wim^2     */
+            sqr_im<N>(s.wim2, s, k);                         /* wim2 = wim^2     */
             s.lazy = false;
         }
     } else {
-        mul_rn<N, true>(s.wim2, s.wim, s.wim, k);            /* wim2 = wim^2     */
+        sqr_im<N>(s.wim2, s, k);                             /* wim2 = wim^2     */
     }
-    mul_rn<N, true>(s.wre2, s.wre, s.wre, k);                /* wre2 = wre^2     */
+    sqr_re<N>(s.wre2, s, k);                                 /* wre2 = wre^2     */
     /* RN(wim2 + wre2) > 4  <=>  wim2 + wre2 > 4 + 2^(2-p) */
     const double thresh = 4.0 + ldexp(1.0, 2 - (32 * N - k));
     return escaped<N>(s.wim2, s.wre2, thresh, k);
@@ -994,6 +1048,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, true>())) void k_rn_op_probe(
     const int fractal = t.fractal;
     for (int32_t wz = 1; wz <= warm; ++wz)
         (void)rn_step<N, true>(s, fractal, wz, 0);
+    rn_words<N>(s);
     const double thresh = 4.0 + ldexp(1.0, 2 - 32 * N);
     uint32_t h = 0;
     mp<N> x = s.wre, y = s.wim;
@@ -1038,6 +1093,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, true>())) void k_rn_op_probe(
             asm volatile("" : "+v"(x.m[0]));
         break;
     }
+    rn_words<N>(s);
     t.out[idx] = h ^ x.m[N - 1] ^ s.wre.m[N - 1] ^ s.wre2.m[N - 1];
 }
 
@@ -1201,6 +1257,7 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
                     load_mp<N>(s.wim, st + MDZG_VS(N));
                     load_mp<N>(s.wre2, st + 2 * MDZG_VS(N));
                     load_mp<N>(s.wim2, st + 3 * MDZG_VS(N));
+                    rn_z<N>(s);
                     s.lazy = false;
                     mp<N> cr, ci;
                     if (tp->family == 1) {
@@ -1277,9 +1334,10 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
                    exact square (wim is the value it squares) */
                 if constexpr (rn_lazy<N, FULL>()) {
                     if (s.lazy)
-                        mul_rn<N, true>(s.wim2, s.wim, s.wim, 0);
+                        sqr_im<N>(s.wim2, s, 0);
                     s.lazy = false;
                 }
+                rn_words<N>(s);
                 uint32_t* st = tp->state + (size_t)local * 4 * MDZG_VS(N);
                 store_mp<N>(st, s.wre);
                 store_mp<N>(st + MDZG_VS(N), s.wim);

@@ -273,9 +273,10 @@ constexpr int cut_words() { return N <= 8 ? 1 : (N <= 16 ? 2 : 4); }
    kclr.  In the kernels the round bit lies in one of the cut_words<N>()
    lowest words, and only those are masked: with masks on every word a
    rounding took more instructions than the addition it followed, and the
-   masks, moved out of the loop, spilled registers in the ragged kernels from
-   10 words up (again() keeps them in).  512x512 frames at 400, 800, 900 and
-   1000 bits: 15.5 -> 9.9, 89.7 -> 45.6, 101 -> 59.6, 80 -> 59.4 ms. */
+   masks, which the compiler moves out of the loop, spilled registers in the
+   ragged kernels from 10 words up.  512x512 frames at 400, 600, 800 and 900
+   bits: 15.5 -> 9.2, 33.5 -> 22.4, 89.7 -> 40.5, 101 -> 52.6 ms (with the
+   limb products). */
 template <int N>
 MP_HD void round_masked(uint32_t* R, uint32_t G, uint32_t S, int32_t& e, int kclr)
 {
@@ -301,7 +302,6 @@ MP_HD void round_masked(uint32_t* R, uint32_t G, uint32_t S, int32_t& e, int kcl
         return;
     }
     constexpr int W = CUTS_BOUNDED && cut_words<N>() < N ? cut_words<N>() : N;
-    kclr = again(kclr);
     const int rw = (kclr - 1) >> 5;                      /* word of the round bit */
     const uint32_t b = (uint32_t)(kclr - 1) & 31u;
     const uint32_t half = 1u << b;
@@ -775,6 +775,153 @@ MP_HD void mant_product(const uint32_t* a, const uint32_t* b, uint32_t* H, uint3
         mant_mul<N, K0>(a, SQR ? a : b, H, S);
 }
 
+/* Short products of wide significands in 29-bit limbs.  In 32-bit words every
+   multiply-accumulate of a column is followed by an add of its carry into the
+   third accumulator word.  Products of 29-bit limbs stay below 2^58, so a
+   64-bit accumulator holds a column's up to 38 of them and the carry adds are
+   gone: one instruction a product instead of two, for (32/29)^2 as many
+   products, two instructions to split a column's sum and about two to put a
+   result word together.  At 32 words the product takes 910 instructions
+   against 1190 and a square 600 against 700, z converted once an iteration;
+   below 20 words the conversions outweigh it.  512x512 frames of a deep zoom
+   at 640, 768 and 1024 bits: 22.5 -> 20.3, 35.1 -> 28.5, 56.4 -> 51.4 ms.
+
+   The columns k < K0 are left out.  Their sum is below K0 2^(29 K0 + 29), less
+   than one unit of the guard word (checked below), so the exact product lies
+   in [H, H + 2) units of H[0], within the window that mul_rn's check allows
+   for the word form. */
+#ifndef MDZG_LIMB_MIN
+#define MDZG_LIMB_MIN 20
+#endif
+template <int N>
+constexpr bool limb_product() { return N >= MDZG_LIMB_MIN; }
+
+static constexpr int LB = 29;
+static constexpr uint32_t LMASK = (1u << LB) - 1u;
+
+template <int N>
+constexpr int limb_count() { return (32 * N + LB - 1) / LB; }
+
+template <int N>
+struct limbs {
+    uint32_t l[limb_count<N>()];
+};
+
+template <int N>
+MP_HD void to_limbs(limbs<N>& x, const uint32_t* m)
+{
+#pragma unroll
+    for (int i = 0; i < limb_count<N>(); ++i) {
+        const int w = (LB * i) >> 5, s = (LB * i) & 31;
+        x.l[i] = (s + LB <= 32 || w + 1 >= N)
+                     ? (m[w] >> s) & LMASK
+                     : funnel_r(w + 1 < N ? m[w + 1] : 0u, m[w], (uint32_t)s) & LMASK;
+    }
+}
+
+/* words [w0, w0 + W) of the number with limbs l0, l0 + 1, ... in L */
+template <int W, int w0, int l0, int NL>
+MP_HD void from_limbs(uint32_t* m, const uint32_t* L)
+{
+#pragma unroll
+    for (int j = 0; j < W; ++j) {
+        const int b = 32 * (w0 + j), i = b / LB - l0, s = b % LB;
+        uint32_t v = L[i] >> s;
+        if (i + 1 < NL) v |= L[i + 1] << (LB - s);
+        if (2 * LB - s < 32 && i + 2 < NL) v |= L[i + 2] << (2 * LB - s);
+        m[j] = v;
+    }
+}
+
+/* x, not before y is known: keeps the scheduler from starting the sums of
+   many columns at once, which fills the registers */
+MP_HD uint32_t after(uint32_t x, uint64_t y)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(x) : "v"(y));
+#endif
+    return x;
+}
+MP_HD uint64_t after(uint64_t x, uint64_t y)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(x) : "v"(y));
+#endif
+    return x;
+}
+
+/* acc += column k of a * b (SQR: a * a) */
+template <int N, bool SQR>
+MP_HD void limb_col(const limbs<N>& a, const limbs<N>& b, int k, uint64_t& acc)
+{
+    constexpr int K = limb_count<N>();
+    const int i0 = k < K ? 0 : k - K + 1, i1 = k < K ? k : K - 1;
+    if (SQR) {
+        uint64_t o = 0;
+#pragma unroll
+        for (int i = i0; 2 * i < k && i <= i1; ++i)
+            o += (uint64_t)(i == i0 ? after(a.l[i], acc) : a.l[i]) * a.l[k - i];
+        if (2 * i0 < k && i0 <= i1) acc += o << 1;
+        if ((k & 1) == 0 && k / 2 < K) acc += (uint64_t)a.l[k / 2] * a.l[k / 2];
+    } else {
+        acc = after(acc, acc);
+#pragma unroll
+        for (int i = i0; i <= i1; ++i) acc += (uint64_t)a.l[i] * b.l[k - i];
+    }
+}
+
+/* limb of the guard word's lowest bit, and that bit's place in it */
+template <int N>
+constexpr int limb_l0() { return 32 * (N - 1) / LB; }
+template <int N>
+constexpr int limb_s0() { return 32 * (N - 1) % LB; }
+
+/* H = the top N+1 words of a * b (SQR: a * a) without the columns below K0 =
+   l0 - 1; low: its bits below H, from column K0 up */
+template <int N, bool SQR>
+MP_HD void limb_mul(const limbs<N>& a, const limbs<N>& b, uint32_t* H, uint64_t& low)
+{
+    constexpr int L0 = limb_l0<N>(), K0 = L0 - 1;
+    constexpr int TOP = (64 * N + LB - 1) / LB;   /* limbs of the whole product */
+    static_assert(limb_count<N>() <= 38 && LB * (K0 + 1) + stages(K0) <= 32 * (N - 1),
+                  "bounds above");
+    uint32_t R[TOP - L0];
+    uint64_t acc = 0;
+#pragma unroll
+    for (int k = K0; k < TOP; ++k) {
+        limb_col<N, SQR>(a, b, k, acc);
+        if (k >= L0)
+            R[k - L0] = (uint32_t)acc & LMASK;
+        else
+            low = (uint32_t)acc & LMASK;
+        acc >>= LB;
+    }
+    low |= (uint64_t)(R[0] & ((1u << limb_s0<N>()) - 1u)) << LB;
+    from_limbs<N + 1, N - 1, L0, TOP - L0>(H, R);
+}
+
+/* the columns that limb_mul left out added to its H and low: H exact, S the
+   sticky bit of everything below */
+template <int N, bool SQR>
+MP_HD void limb_rest(const limbs<N>& a, const limbs<N>& b, uint32_t* H, uint64_t low, uint32_t& S)
+{
+    uint64_t acc = 0;
+    uint32_t st = 0;
+#pragma unroll
+    for (int k = 0; k < limb_l0<N>() - 1; ++k) {
+        limb_col<N, SQR>(a, b, k, acc);
+        st |= (uint32_t)acc & LMASK;
+        acc >>= LB;
+    }
+    acc += low;
+    constexpr int W = LB + limb_s0<N>();
+    S = (uint32_t)((st != 0) | ((acc & (((uint64_t)1 << W) - 1u)) != 0));
+    uint32_t c;
+    H[0] = add_cc(H[0], (uint32_t)(acc >> W), 0u, c);
+#pragma unroll
+    for (int j = 1; j <= N; ++j) H[j] = add_cc(H[j], 0u, c, c);
+}
+
 /* product of normalised values is >= 2^(64N-2): at most one left shift,
    skipped by a wave none of whose lanes needs it */
 template <int N>
@@ -790,42 +937,114 @@ MP_HD void norm_product(uint32_t* H, int32_t& e)
     }
 }
 
-/* r = RN_p(a * b) (SQR: b ignored, a*a) */
-template <int N, bool SQR>
-MP_HD void mul_rn(mp<N>& r, const mp<N>& a, const mp<N>& b, int kclr)
+/* the limbs of a value beside its exponent and sign: what a product of
+   wide significands reads */
+template <int N>
+struct limb_value {
+    limbs<N> m;
+    int32_t e;
+    uint32_t s;
+};
+
+template <int N>
+MP_HD void to_limbs(limb_value<N>& x, const mp<N>& a)
 {
-    constexpr int K0 = short_col<N>();
-    uint32_t H[N + 1];
-    uint32_t S;
-    mant_product<N, SQR, K0>(a.m, b.m, H, S);
-    const int32_t e0 = SQR ? (a.e + a.e) : (a.e + b.e);
-    int32_t e = e0;
-    const uint32_t s = SQR ? 0u : (a.s ^ b.s);
-    norm_product<N>(H, e);
-    if (K0 > 0) {
-        constexpr uint32_t U = 2u * N;
-        const bool unsure = (kclr == 0) ? ((uint32_t)(0x80000000u - H[0]) < U)
-                                        : ((uint32_t)(H[0] + (U - 1u)) < U);
-        S = 1;
-        /* marked unlikely, the exact product is laid out past the kernel's
-           loops, which keeps the loop's instructions contiguous.  Placed
-           between them (the compiler's choice without the mark), the
-           exact products left the 1024-bit loop with 1.2e8
-           instruction-cache misses on a 737,280-pixel band against 6e4
-           out of line, and 15 % slower. */
-        if (__builtin_expect(wave_any(unsure), 0)) {
-            MDZG_NOTE_SHORT_FALLBACK();
-            mant_product<N, SQR, 0>(a.m, b.m, H, S);
-            e = e0;
-            norm_product<N>(H, e);
-        }
-    }
+    to_limbs<N>(x.m, a.m);
+    x.e = a.e;
+    x.s = a.s;
+}
+
+template <int N>
+MP_HD void from_limbs(mp<N>& a, const limb_value<N>& x)
+{
+    from_limbs<N, 0, 0, limb_count<N>()>(a.m, x.m.l);
+    a.e = x.e;
+    a.s = x.s;
+}
+
+/* true where the window of a short product with guard word G may reach a
+   midpoint (N >= MDZG_SHORT_MIN, above) */
+template <int N>
+MP_HD bool short_unsure(uint32_t G, int kclr)
+{
+    constexpr uint32_t U = 2u * N;
+    return (kclr == 0) ? ((uint32_t)(0x80000000u - G) < U) : ((uint32_t)(G + (U - 1u)) < U);
+}
+
+/* r = the rounded product of exponent e and sign s from its normalised top
+   words H and sticky bit S */
+template <int N>
+MP_HD void round_product(mp<N>& r, uint32_t* H, uint32_t S, int32_t e, uint32_t s, int kclr)
+{
     round_p<N>(H + 1, H[0], S, e, kclr);
     const bool z = (H[N] == 0);
 #pragma unroll
     for (int j = 0; j < N; ++j) r.m[j] = H[j + 1];
     r.e = z ? EZERO : e;
     r.s = z ? 0u : s;
+}
+
+/* r = RN_p(a * b) (SQR: b ignored, a*a) of operands in limbs */
+template <int N, bool SQR>
+MP_HD void mul_limbs(mp<N>& r, const limb_value<N>& a, const limb_value<N>& b, int kclr)
+{
+    uint32_t H[N + 1];
+    uint32_t S = 1;
+    uint64_t low = 0;
+    limb_mul<N, SQR>(a.m, SQR ? a.m : b.m, H, low);
+    const int32_t e0 = SQR ? (a.e + a.e) : (a.e + b.e);
+    int32_t e = e0;
+    norm_product<N>(H, e);
+    if (__builtin_expect(wave_any(short_unsure<N>(H[0], kclr)), 0)) {
+        MDZG_NOTE_SHORT_FALLBACK();
+        /* from the short product itself, the normalising shift undone: the
+           exact product from the words would need both forms of the operands */
+        const uint32_t un = (uint32_t)(e0 - e);
+#pragma unroll
+        for (int j = 0; j < N; ++j) H[j] = un ? funnel_r(H[j + 1], H[j], 1u) : H[j];
+        H[N] >>= un;
+        limb_rest<N, SQR>(a.m, SQR ? a.m : b.m, H, low, S);
+        e = e0;
+        norm_product<N>(H, e);
+    }
+    round_product<N>(r, H, S, e, SQR ? 0u : (a.s ^ b.s), kclr);
+}
+
+/* r = RN_p(a * b) (SQR: b ignored, a*a) */
+template <int N, bool SQR>
+MP_HD void mul_rn(mp<N>& r, const mp<N>& a, const mp<N>& b, int kclr)
+{
+    if constexpr (limb_product<N>()) {
+        limb_value<N> la, lb;
+        to_limbs<N>(la, a);
+        if (!SQR) to_limbs<N>(lb, b);
+        mul_limbs<N, SQR>(r, la, SQR ? la : lb, kclr);
+    } else {
+        constexpr int K0 = short_col<N>();
+        uint32_t H[N + 1];
+        uint32_t S;
+        mant_product<N, SQR, K0>(a.m, b.m, H, S);
+        const int32_t e0 = SQR ? (a.e + a.e) : (a.e + b.e);
+        int32_t e = e0;
+        norm_product<N>(H, e);
+        if (K0 > 0) {
+            const bool unsure = short_unsure<N>(H[0], kclr);
+            S = 1;
+            /* marked unlikely, the exact product is laid out past the kernel's
+               loops, which keeps the loop's instructions contiguous.  Placed
+               between them (the compiler's choice without the mark), the
+               exact products left the 1024-bit loop with 1.2e8
+               instruction-cache misses on a 737,280-pixel band against 6e4
+               out of line, and 15 % slower. */
+            if (__builtin_expect(wave_any(unsure), 0)) {
+                MDZG_NOTE_SHORT_FALLBACK();
+                mant_product<N, SQR, 0>(a.m, b.m, H, S);
+                e = e0;
+                norm_product<N>(H, e);
+            }
+        }
+        round_product<N>(r, H, S, e, SQR ? 0u : (a.s ^ b.s), kclr);
+    }
 }
 
 /* ------------------------------------------------------------------ */
