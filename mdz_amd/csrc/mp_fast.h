@@ -689,11 +689,13 @@ struct rn_form {
     uint32_t va;                  /* 1: hybrid                                */
 };
 
-/* an iteration's operand as loaded: a zero's exponent raised to EZF */
+/* an operand as loaded: a zero's exponent raised to EZF.  A sum with a zero c
+   (a Julia set of c = 0) then flushes values below 2^EZF, whose squares'
+   exponents would otherwise pass the end of an int32 after 30 iterations. */
 template <int N>
 MP_HD void clamp_zero(mp<N>& v)
 {
-    if (rn_fast<N>() && is_zero<N>(v))
+    if (is_zero<N>(v))
         v.e = EZF;
 }
 
