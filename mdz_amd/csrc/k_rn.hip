@@ -1,7 +1,10 @@
 /* k_rn.hip -- the RN<N> kernels of k_escape.h for one word count, selected by
  * -DMDZG_N=<N> at compile time (one object per N, built in parallel).
- * Exports mdzg_kget_rn<N>(full, &tile, &persist, &slice) to the launch table. */
+ * Exports mdzg_kget_rn<N>(full, &tile, &persist, &slice) and, for the
+ * four-lanes-a-pixel forms, mdzg_kquad_rn<N>(full, &persist, &slice) to the
+ * launch table. */
 #include "k_escape.h"
+#include "k_quad.h"
 
 #ifndef MDZG_N
 #error "build with -DMDZG_N=<words>"
@@ -9,6 +12,23 @@
 
 #define KGET_NAME2(n) mdzg_kget_rn##n
 #define KGET_NAME(n) KGET_NAME2(n)
+#define KQUAD_NAME2(n) mdzg_kquad_rn##n
+#define KQUAD_NAME(n) KQUAD_NAME2(n)
+
+extern "C" void KQUAD_NAME(MDZG_N)(int full, const void** persist, const void** slice)
+{
+    *persist = *slice = nullptr;
+#if MDZG_N >= 10
+    static_assert(rn_quad<MDZG_N>(), "the word counts of k_quad.h");
+    if (full) {
+        *persist = (const void*)k_rn_quad<MDZG_N, true>;
+        *slice = (const void*)k_rn_quad_slice<MDZG_N, true>;
+    } else {
+        *persist = (const void*)k_rn_quad<MDZG_N, false>;
+        *slice = (const void*)k_rn_quad_slice<MDZG_N, false>;
+    }
+#endif
+}
 
 extern "C" void KGET_NAME(MDZG_N)(int full, const void** tile, const void** persist,
                                   const void** slice)

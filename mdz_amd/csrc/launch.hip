@@ -29,6 +29,22 @@ void mdzg_kget_rn20(int, const void**, const void**, const void**);
 void mdzg_kget_rn24(int, const void**, const void**, const void**);
 void mdzg_kget_rn28(int, const void**, const void**, const void**);
 void mdzg_kget_rn32(int, const void**, const void**, const void**);
+void mdzg_kquad_rn1(int, const void**, const void**);
+void mdzg_kquad_rn2(int, const void**, const void**);
+void mdzg_kquad_rn3(int, const void**, const void**);
+void mdzg_kquad_rn4(int, const void**, const void**);
+void mdzg_kquad_rn5(int, const void**, const void**);
+void mdzg_kquad_rn6(int, const void**, const void**);
+void mdzg_kquad_rn7(int, const void**, const void**);
+void mdzg_kquad_rn8(int, const void**, const void**);
+void mdzg_kquad_rn10(int, const void**, const void**);
+void mdzg_kquad_rn12(int, const void**, const void**);
+void mdzg_kquad_rn14(int, const void**, const void**);
+void mdzg_kquad_rn16(int, const void**, const void**);
+void mdzg_kquad_rn20(int, const void**, const void**);
+void mdzg_kquad_rn24(int, const void**, const void**);
+void mdzg_kquad_rn28(int, const void**, const void**);
+void mdzg_kquad_rn32(int, const void**, const void**);
 void mdzg_kget_gmp(int bucket, const void**, const void**, const void**);
 const void* mdzg_kprobe_rn4(void);
 const void* mdzg_kprobe_rn32(void);
@@ -41,6 +57,13 @@ static const kget_fn kget_rn[MDZG_NCLASS_N] = {
     mdzg_kget_rn10, mdzg_kget_rn12, mdzg_kget_rn14, mdzg_kget_rn16,
     mdzg_kget_rn20, mdzg_kget_rn24, mdzg_kget_rn28, mdzg_kget_rn32,
 };
+typedef void (*kquad_fn)(int, const void**, const void**);
+static const kquad_fn kquad_rn[MDZG_NCLASS_N] = {
+    mdzg_kquad_rn1,  mdzg_kquad_rn2,  mdzg_kquad_rn3,  mdzg_kquad_rn4,
+    mdzg_kquad_rn5,  mdzg_kquad_rn6,  mdzg_kquad_rn7,  mdzg_kquad_rn8,
+    mdzg_kquad_rn10, mdzg_kquad_rn12, mdzg_kquad_rn14, mdzg_kquad_rn16,
+    mdzg_kquad_rn20, mdzg_kquad_rn24, mdzg_kquad_rn28, mdzg_kquad_rn32,
+};
 static const int rn_kid[MDZG_NCLASS_N] = MDZG_RN_KID_INIT;
 
 /* RN class of an RN kernel id */
@@ -52,12 +75,21 @@ static int class_of_kid(int kid)
     return i;
 }
 
-/* form: 0 = per-tile, 1 = persistent, 2 = resumable slice */
+/* form: 0 = per-tile, 1 = persistent, 2 = resumable slice, 3 and 4 = persistent
+   and slice with four lanes a pixel (null where a kernel has none) */
 static void lookup(int kid, int form, const void** f)
 {
     const void* t = nullptr;
     const void* p = nullptr;
     const void* sl = nullptr;
+    if (form >= 3) {
+        *f = nullptr;
+        if (kid == 0 || (kid >= MDZG_KID_GMP0 && kid < MDZG_KID_GMP0 + MDZG_NGMP))
+            return;
+        kquad_rn[class_of_kid(kid)]((kid - 1) & 1, &p, &sl);
+        *f = form == 3 ? p : sl;
+        return;
+    }
     if (kid == 0)
         mdzg_kget_fp64(&t, &p, &sl);
     else if (kid >= MDZG_KID_GMP0 && kid < MDZG_KID_GMP0 + MDZG_NGMP)
@@ -134,6 +166,29 @@ extern "C" {
 
 int mdzg_dev_nkernels(void) { return MDZG_NKERNELS; }
 
+/* Four lanes a pixel (k_quad.h) up to two of its waves per SIMD, 32768 pixels
+   on 256 CUs.  Times of a deep zoom, one lane a pixel / four, up to one wave
+   per SIMD of the latter (128x128) and up to two (181x181): 1024 bits 17.2 /
+   8.5 and 13.2 ms, 512 bits 4.30 / 2.56 and 3.65, 320 bits 1.69 / 1.24 and
+   1.58; with more (221x221) 17.9, 4.97 and 2.12 ms, slower than one lane. */
+int mdzg_dev_quad_pays(int kid, uint64_t total, int ncu)
+{
+    if (kid < 0 || kid >= mdzg_dev_nkernels() || total > (uint64_t)ncu * 128u)
+        return 0;
+    const void* f;
+    lookup(kid, 3, &f);
+    return f != nullptr;
+}
+
+/* blocks of a persistent (slice) launch: one lane a pixel, four with quad,
+   at most blocks_per_cu a CU */
+int mdzg_dev_grid(uint64_t total, int quad, int ncu, int blocks_per_cu)
+{
+    const uint64_t want = ((quad ? 4 * total : total) + 255) / 256;
+    const uint64_t cap = (uint64_t)ncu * (uint64_t)(blocks_per_cu > 0 ? blocks_per_cu : 1);
+    return (int)(want < cap ? (want ? want : 1) : cap);
+}
+
 /* kind 0: v_mad_u64_u32, 1: v_fma_f64.  blocks of 256 lanes (4 waves, one
    per SIMD) per CU x ncu, iters x 4 instructions per lane; *ms the kernel
    time by HIP events on a stream of its own. */
@@ -185,12 +240,14 @@ int mdzg_dev_node_fill(mdzg_gnode* n, uint32_t* p, uint64_t count, uint32_t v)
 
 int mdzg_dev_node_persist(mdzg_gnode* n, int kid, const mdzg_dtile* d_tiles, int ntiles,
                           uint64_t total, unsigned long long* d_counter, const int* d_cancel,
-                          int grid, int chunk)
+                          int quad, int grid, int chunk)
 {
     if (!n || kid < 0 || kid >= mdzg_dev_nkernels() || ntiles <= 0 || grid <= 0 || chunk <= 0)
         return -1;
     const void* f;
-    lookup(kid, 1, &f);
+    lookup(kid, quad ? 3 : 1, &f);
+    if (!f)
+        return -1;
     node_init(n, f, (unsigned)grid, 256);
     node_arg(n, d_tiles);
     node_arg(n, ntiles);
@@ -202,14 +259,16 @@ int mdzg_dev_node_persist(mdzg_gnode* n, int kid, const mdzg_dtile* d_tiles, int
 }
 
 int mdzg_dev_node_slice(mdzg_gnode* n, int kid, const mdzg_dtile* d_tiles, int ntiles,
-                        uint64_t total, unsigned long long* d_counter, int grid, int budget,
-                        int lane_budget)
+                        uint64_t total, unsigned long long* d_counter, int quad, int grid,
+                        int budget, int lane_budget)
 {
     if (!n || kid < 0 || kid >= mdzg_dev_nkernels() || ntiles <= 0 || grid <= 0 || budget <= 0 ||
         lane_budget <= 0)
         return -1;
     const void* f;
-    lookup(kid, 2, &f);
+    lookup(kid, quad ? 4 : 2, &f);
+    if (!f)
+        return -1;
     node_init(n, f, (unsigned)grid, 256);
     node_arg(n, d_tiles);
     node_arg(n, ntiles);
@@ -227,6 +286,8 @@ int mdzg_dev_occupancy(int kid, int persist)
     const void* f;
     lookup(kid, persist, &f);
     int nb = 0;
+    if (!f)
+        return 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 256, 0) != hipSuccess)
         return 0;
     return nb;
@@ -257,13 +318,15 @@ int mdzg_dev_launch_op_probe(int nwords, const mdzg_dtile* d_tile, uint32_t npix
 }
 
 int mdzg_dev_launch_persist(int kid, const mdzg_dtile* d_tiles, int ntiles, uint64_t total,
-                            unsigned long long* d_counter, const int* d_cancel, int grid,
-                            int chunk, hipStream_t st)
+                            unsigned long long* d_counter, const int* d_cancel, int quad,
+                            int grid, int chunk, hipStream_t st)
 {
     if (kid < 0 || kid >= mdzg_dev_nkernels() || ntiles <= 0 || grid <= 0 || chunk <= 0)
         return -1;
     const void* f;
-    lookup(kid, 1, &f);
+    lookup(kid, quad ? 3 : 1, &f);
+    if (!f)
+        return -1;
     void* args[] = { (void*)&d_tiles, (void*)&ntiles, (void*)&total, (void*)&d_counter,
                      (void*)&d_cancel, (void*)&chunk };
     return hipLaunchKernel(f, dim3(grid), dim3(256), args, 0, st) == hipSuccess ? 0 : -3;
@@ -279,20 +342,6 @@ int mdzg_dev_occupancy_slice(int kid)
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, 256, 0) != hipSuccess)
         return 0;
     return nb;
-}
-
-int mdzg_dev_launch_slice(int kid, const mdzg_dtile* d_tiles, int ntiles, uint64_t total,
-                          unsigned long long* d_counter, int grid, int budget, int lane_budget,
-                          hipStream_t st)
-{
-    if (kid < 0 || kid >= mdzg_dev_nkernels() || ntiles <= 0 || grid <= 0 || budget <= 0 ||
-        lane_budget <= 0)
-        return -1;
-    const void* f;
-    lookup(kid, 2, &f);
-    void* args[] = { (void*)&d_tiles, (void*)&ntiles, (void*)&total, (void*)&d_counter,
-                     (void*)&budget, (void*)&lane_budget };
-    return hipLaunchKernel(f, dim3(grid), dim3(256), args, 0, st) == hipSuccess ? 0 : -3;
 }
 
 } /* extern "C" */

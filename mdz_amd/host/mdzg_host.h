@@ -17,11 +17,15 @@
 
 /* kernel table (launch.hip) */
 int mdzg_dev_nkernels(void);
-int mdzg_dev_occupancy(int kid, int persist);
+/* form: 0 per tile, 1 persistent, 2 slice, 3 / 4 with four lanes a pixel (0 blocks
+   where the kernel has no such form) */
+int mdzg_dev_occupancy(int kid, int form);
+int mdzg_dev_quad_pays(int kid, uint64_t total, int ncu);
+int mdzg_dev_grid(uint64_t total, int quad, int ncu, int blocks_per_cu);
 int mdzg_dev_launch_tile(int kid, const mdzg_dtile* d_tile, uint32_t npix, hipStream_t st);
 int mdzg_dev_launch_persist(int kid, const mdzg_dtile* d_tiles, int ntiles, uint64_t total,
-                            unsigned long long* d_counter, const int* d_cancel, int grid,
-                            int chunk, hipStream_t st);
+                            unsigned long long* d_counter, const int* d_cancel, int quad,
+                            int grid, int chunk, hipStream_t st);
 int mdzg_dev_occupancy_slice(int kid);
 int mdzg_dev_rate_probe(int kind, int ncu, int blocks_per_cu, int iters, double* ms);
 int mdzg_dev_launch_op_probe(int nwords, const mdzg_dtile* d_tile, uint32_t npix, int op,
@@ -30,10 +34,10 @@ int mdzg_dev_launch_op_probe(int nwords, const mdzg_dtile* d_tile, uint32_t npix
 int mdzg_dev_node_fill(mdzg_gnode* n, uint32_t* p, uint64_t count, uint32_t v);
 int mdzg_dev_node_persist(mdzg_gnode* n, int kid, const mdzg_dtile* d_tiles, int ntiles,
                           uint64_t total, unsigned long long* d_counter, const int* d_cancel,
-                          int grid, int chunk);
+                          int quad, int grid, int chunk);
 int mdzg_dev_node_slice(mdzg_gnode* n, int kid, const mdzg_dtile* d_tiles, int ntiles,
-                        uint64_t total, unsigned long long* d_counter, int grid, int budget,
-                        int lane_budget);
+                        uint64_t total, unsigned long long* d_counter, int quad, int grid,
+                        int budget, int lane_budget);
 int mdzg_dev_node_colour(mdzg_gnode* node, const uint32_t* counts, int real_w, int user_w,
                          int user_h, int aa, const uint32_t* palette, int n, int offset,
                          double sc, int ip, uint32_t depth, uint32_t* rgb,
@@ -45,9 +49,6 @@ void mdzg_gcache_destroy(mdzg_gcache* gc);
 void mdzg_gcache_counts(mdzg_gcache* gc, uint64_t* hits, uint64_t* builds);
 int mdzg_graph_run(mdzg_gcache* gc, const mdzg_gnode* root, const mdzg_gnode* par, int npar,
                    const mdzg_gnode* tail, hipStream_t st);
-int mdzg_dev_launch_slice(int kid, const mdzg_dtile* d_tiles, int ntiles, uint64_t total,
-                          unsigned long long* d_counter, int grid, int budget, int lane_budget,
-                          hipStream_t st);
 
 /* k_colour.hip: counts -> RGB (palette_apply / do_anti_aliasing), adding the
    pixel-iterations of the counts read to *iters when iters is not null; at
@@ -128,6 +129,7 @@ struct mdzg_ctx {
     hipStream_t ctl;            /* cancel-flag writes */
     int* d_cancel_zero;         /* a device int that stays 0 */
     int occ[MDZG_NKERNELS];     /* resident blocks per CU (persistent grid) */
+    int occ_quad[MDZG_NKERNELS];   /* the same of the four-lane form, 0: none */
     int chunk[MDZG_NKERNELS];   /* iterations between lane refills */
     pthread_mutex_t lock;
     /* mdzg_render_tile_noalloc: the device address of the library's static
@@ -148,6 +150,7 @@ struct mdzg_ctx {
        mdzg_create; 0 = never) */
     long fail_plan;
     long plans;
+    int jobs;                   /* launched and not yet waited for */
 };
 
 /* noalloc.hip: device address of the static scratch array of the current

@@ -105,6 +105,7 @@ struct mdzg_server {
     hipEvent_t ev_fork, ev_join[MAX_KID];
 
     int occ_slice[MAX_KID];
+    int occ_quad[MAX_KID];      /* four-lane slices, 0: none */
     long long budget_pix[MAX_KID];
     long long act_pix[MAX_KID];
     int slice_iters[MAX_KID];
@@ -430,13 +431,12 @@ static int run_slice(mdzg_server* s)
     for (int k = 0; k < MAX_KID; ++k) {
         if (!cnt[k])
             continue;
-        const uint64_t cap = (uint64_t)c->ncu * (uint64_t)s->occ_slice[k];
-        const uint64_t want = (total[k] + 255) / 256;
-        int grid = (int)(want < cap ? want : cap);
-        if (grid < 1) grid = 1;
+        const int quad = s->occ_quad[k] > 0 && mdzg_dev_quad_pays(k, total[k], c->ncu);
+        const int grid = mdzg_dev_grid(total[k], quad, c->ncu,
+                                       quad ? s->occ_quad[k] : s->occ_slice[k]);
         const int it = s->slice_iters[k];
         if (mdzg_dev_node_slice(&par[nk++], k, s->d_desc + first[k], cnt[k], total[k],
-                                s->d_ctr + k, grid, lane_cap[k] ? INT32_MAX : it,
+                                s->d_ctr + k, quad, grid, lane_cap[k] ? INT32_MAX : it,
                                 lane_cap[k] ? 2 * it : INT32_MAX) != 0)
             return MDZG_ERR_DEVICE;
     }
@@ -754,6 +754,7 @@ int mdzg_server_create(mdzg_ctx* ctx, const mdzg_server_cfg* cfg, mdzg_server** 
             s->occ_slice[k] = mdzg_dev_occupancy_slice(k);
             if (s->occ_slice[k] < 1)
                 s->occ_slice[k] = 1;
+            s->occ_quad[k] = mdzg_dev_occupancy(k, 4);
             const int lanes = ctx->ncu * s->occ_slice[k] * 256;
             s->budget_pix[k] = (long long)(s->cfg.occupancy_budget * (double)lanes);
             int nw = mdzg_kid_words(k);
