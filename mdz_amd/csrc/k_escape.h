@@ -900,17 +900,17 @@ __device__ __forceinline__ bool rn_step(rn_state<N>& s, int fractal, int32_t wz,
     return escaped<N>(s.wim2, s.wre2, thresh, k);
 }
 
-/* Iterations between comparisons of the RN loops of up to 8 words (about 25
-   instructions in 32 iterations of 200 to 530).  The kept z lies in the
+/* Iterations between comparisons of the RN loops of mp_fast.h (about 25
+   instructions in 32 iterations of 200 to 730).  The kept z lies in the
    block's LDS, word w of lane t at [w][t]: both significands, then the
    exponents with their signs.  The wider loops make none: views that need
    them lie too deep for p / -log2 |multiplier| iterations to be few. */
 #define MDZG_CYCLE_RN 32
 
-template <int N>
+template <int N, bool FULL>
 constexpr int cycle_words()
 {
-    return rn_fast<N>() ? 2 * N + 2 : 0;
+    return rn_fast<N, FULL>() ? 2 * N + 2 : 0;
 }
 
 /* true on the lanes of `on` whose orbit is periodic; k counts a lane's
@@ -979,14 +979,14 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_tile(cons
         return;
     const int row = (int)(idx / (uint32_t)t.ncols), col = (int)(idx % (uint32_t)t.ncols);
     __shared__ uint32_t c_lds[c_in_lds<N>() ? 2 * (N + 2) * 256 : 1];
-    __shared__ uint32_t kept[cycle_words<N>() * 256 + 1];
+    __shared__ uint32_t kept[cycle_words<N, FULL>() * 256 + 1];
     rn_state<N> s;
     s.c.init(c_lds);
     rn_init<N, FULL>(s, t, row, col);
     const int fractal = t.fractal, kclr = t.kclr;
     const int32_t depth = t.depth;
     uint32_t count = 0;
-    if constexpr (rn_fast<N>()) {
+    if constexpr (rn_fast<N, FULL>()) {
         rn_prec<FULL> pr;
         set_prec(pr, kclr);
         const rn_form fm = form_of(fractal);
@@ -1123,7 +1123,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
     set_prec(pr, 0);
     int rem = 0, since = 0;
     uint32_t seen = 0;
-    __shared__ uint32_t kept[cycle_words<N>() * 256 + 1];
+    __shared__ uint32_t kept[cycle_words<N, FULL>() * 256 + 1];
     const bool by_lane = N < 24 && total <= (uint64_t)gridDim.x * blockDim.x;
     if (by_lane) {
         run.base = (uint64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
@@ -1147,7 +1147,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
                 wz = 0;
                 active = true;
                 asm volatile("" ::"v"(fractal), "v"(kclr), "v"(depth), "v"(out));
-                if constexpr (rn_fast<N>()) {
+                if constexpr (rn_fast<N, FULL>()) {
                     fm = form_of(fractal);
                     set_prec(pr, kclr);
                     seen = 0;
@@ -1159,7 +1159,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
         if (!__any(active))
             break;
         const int stop = ((++round & 15) == 0) ? read_cancel(cancel) : 0;
-        if constexpr (rn_fast<N>()) {
+        if constexpr (rn_fast<N, FULL>()) {
             /* no active lane reaches its depth within rem iterations: lanes
                that finish leave it a bound, a refill (rem = 0) does not */
             if (rem < chunk)
@@ -1228,7 +1228,7 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
     set_prec(pr, 0);
     int since = 0;
     uint32_t seen = 0;
-    __shared__ uint32_t kept[cycle_words<N>() * 256 + 1];
+    __shared__ uint32_t kept[cycle_words<N, FULL>() * 256 + 1];
     bool drained = false;
     wave_run run = { 0, 0u };
     /* the claim loop runs until the wave holds a pixel or the queue is
@@ -1274,7 +1274,7 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
                 depth = tp->depth;
                 left = budget;
                 active = true;
-                if constexpr (rn_fast<N>()) {
+                if constexpr (rn_fast<N, FULL>()) {
                     fm = form_of(fractal);
                     set_prec(pr, kclr);
                     seen = 0;
@@ -1285,7 +1285,7 @@ __global__ __launch_bounds__(256, (rn_min_waves_slice<N, FULL>())) void k_rn_sli
         } while (!__any(active));
         if (!__any(active))
             break;
-        if constexpr (rn_fast<N>()) {
+        if constexpr (rn_fast<N, FULL>()) {
             /* a run that no lane's depth or budget ends: as in k_rn_persist,
                at most 8 iterations between claims */
             const int32_t mine = left < lb ? left : lb;

@@ -1,8 +1,8 @@
 #ifndef MDZG_K_QUAD_H
 #define MDZG_K_QUAD_H
 /*
- * k_quad.h -- four lanes a pixel for the RN loops of 10 words and more, for
- * launches that leave most of the chip idle.
+ * k_quad.h -- four lanes a pixel for the RN loops of 10 words (ragged) and more,
+ * for launches that leave most of the chip idle.
  *
  * A lane that has a pixel to itself issues one instruction per 4.5 cycles
  * however empty the chip is: 7,500 cycles an iteration at 512 bits, 16,700 at
@@ -21,8 +21,8 @@
  *   exchange   quad_perm moves (DPP), one instruction a word
  *
  * About 0.45 of the instructions in a lane's iteration, for four times the
- * lanes: 64x64 tiles at 320, 512 and 1024 bits take 1.13, 2.48 and 8.4 ms
- * against 1.63, 4.35 and 16.7 with one lane a pixel.  Up to 32768 pixels
+ * lanes: 64x64 tiles at 300, 512 and 1024 bits take 1.18, 2.48 and 8.4 ms
+ * against 1.95, 4.35 and 16.7 with one lane a pixel.  Up to 32768 pixels
  * (rule and figures: mdzg_dev_quad_pays).
  *
  * The loop's state between iterations: v = z (wim on q0, wre on q2) and p =
@@ -33,8 +33,11 @@
  */
 #include "k_escape.h"
 
-template <int N>
-constexpr bool rn_quad() { return N >= 10; }
+/* not where the one-lane loop has few votes (mp_fast.h): at 320 bits that
+   takes 1.16 ms for the 256x256 pixels of a wave per SIMD, four lanes 1.24 for
+   128x128 */
+template <int N, bool FULL>
+constexpr bool rn_quad() { return N >= 10 && !rn_fast<N, FULL>(); }
 
 /* lane `p_q` of each quad to lane q */
 template <int P0, int P1, int P2, int P3>

@@ -19,13 +19,16 @@ extern "C" void KQUAD_NAME(MDZG_N)(int full, const void** persist, const void** 
 {
     *persist = *slice = nullptr;
 #if MDZG_N >= 10
-    static_assert(rn_quad<MDZG_N>(), "the word counts of k_quad.h");
     if (full) {
-        *persist = (const void*)k_rn_quad<MDZG_N, true>;
-        *slice = (const void*)k_rn_quad_slice<MDZG_N, true>;
+        if constexpr (rn_quad<MDZG_N, true>()) {
+            *persist = (const void*)k_rn_quad<MDZG_N, true>;
+            *slice = (const void*)k_rn_quad_slice<MDZG_N, true>;
+        }
     } else {
-        *persist = (const void*)k_rn_quad<MDZG_N, false>;
-        *slice = (const void*)k_rn_quad_slice<MDZG_N, false>;
+        if constexpr (rn_quad<MDZG_N, false>()) {
+            *persist = (const void*)k_rn_quad<MDZG_N, false>;
+            *slice = (const void*)k_rn_quad_slice<MDZG_N, false>;
+        }
     }
 #endif
 }

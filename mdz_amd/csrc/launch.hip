@@ -169,8 +169,8 @@ int mdzg_dev_nkernels(void) { return MDZG_NKERNELS; }
 /* Four lanes a pixel (k_quad.h) up to two of its waves per SIMD, 32768 pixels
    on 256 CUs.  Times of a deep zoom, one lane a pixel / four, up to one wave
    per SIMD of the latter (128x128) and up to two (181x181): 1024 bits 17.2 /
-   8.5 and 13.2 ms, 512 bits 4.30 / 2.56 and 3.65, 320 bits 1.69 / 1.24 and
-   1.58; with more (221x221) 17.9, 4.97 and 2.12 ms, slower than one lane. */
+   8.5 and 13.2 ms, 512 bits 4.30 / 2.56 and 3.65, 300 bits 1.96 / 1.25 and
+   1.70; with more (221x221) 17.9, 4.97 and 2.14 ms, slower than one lane. */
 int mdzg_dev_quad_pays(int kid, uint64_t total, int ncu)
 {
     if (kid < 0 || kid >= mdzg_dev_nkernels() || total > (uint64_t)ncu * 128u)

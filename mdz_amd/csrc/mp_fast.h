@@ -1,6 +1,6 @@
 /*
- * mp_fast.h -- the escape loop's iteration for up to 8 words (p <= 256) with
- * few branches.
+ * mp_fast.h -- the escape loop's iteration for up to 8 words (p <= 256), and
+ * for 10 whole ones (p = 320), with few branches.
  *
  * add_rn and mul_rn (mp_rn.h) skip every step that no lane of the wave needs
  * behind a wave vote: about 30 votes an iteration.  With several waves per SIMD
@@ -37,8 +37,10 @@
  *   176 bits   4369 -> 2279       89 -> 102
  *   256 bits   3967 -> 2740       83 -> 81 (frames of escaping pixels: 75 -> 78)
  * What is left is VALU issue: 301 instructions an iteration at 4 words, 39 of
- * them multiply-accumulates.  From 10 words up the products outweigh the
- * votes, and those kernels keep add_rn and mul_rn.
+ * them multiply-accumulates.  At 320 bits an iteration alone takes 3,300
+ * cycles against 4,800 (a 480x360 frame of a saved scene 26.1 -> 21.3 ms); the
+ * ragged 10-word kernel, whose cut may lie in the second word, and those from
+ * 12 words up, where the products outweigh the votes, keep add_rn and mul_rn.
  *
  * A precision of p = 32N - kclr bits with 0 <= kclr < 32 is covered: rounding
  * at bit kclr of the lowest word is one add with carry and a mask.
@@ -54,8 +56,8 @@
 namespace mdzg {
 
 /* word counts whose kernels use these forms */
-template <int N>
-constexpr bool rn_fast() { return N <= 8; }
+template <int N, bool FULL>
+constexpr bool rn_fast() { return N <= 8 || (N == 10 && FULL); }
 
 /* exponent of a zero that enters an iteration: twice it, and its distance to
    any other, fit an int32 */
@@ -212,10 +214,10 @@ MP_HD void sum_words<5>(uint32_t* A, uint32_t* B, uint32_t mA, uint32_t mB, lane
 template <int W>
 MP_HD void sum_chain(uint32_t* A, uint32_t* B, uint32_t mA, uint32_t mB, lanes& c)
 {
-    constexpr int K = W <= 5 ? W : (W + 1) / 2;
+    constexpr int K = W <= 5 ? W : (W <= 10 ? (W + 1) / 2 : 4);
     sum_words<K>(A, B, mA, mB, c);
     if constexpr (W > K)
-        sum_words<W - K>(A + K, B + K, mA, mB, c);
+        sum_chain<W - K>(A + K, B + K, mA, mB, c);
 }
 
 /* H (N+1 words) <<= 1 and e -= 1 on the lanes whose top bit is clear, under
@@ -369,6 +371,30 @@ MP_HD void norm1<8>(uint32_t* H, int32_t& e)
         "v_add_u32 %9, -1, %9\n\t"
         "s_mov_b64 exec, %10"
         : "+&v"(H[0]), "+&v"(H[1]), "+&v"(H[2]), "+&v"(H[3]), "+&v"(H[4]), "+&v"(H[5]), "+&v"(H[6]), "+&v"(H[7]), "+&v"(H[8]),
+          "+&v"(e), "=&s"(sv)
+        :
+        : "vcc");
+}
+template <>
+MP_HD void norm1<10>(uint32_t* H, int32_t& e)
+{
+    uint64_t sv;
+    asm("s_mov_b64 %12, exec\n\t"
+        "v_cmpx_le_i32 vcc, 0, %10\n\t"
+        "v_alignbit_b32 %10, %10, %9, 31\n\t"
+        "v_alignbit_b32 %9, %9, %8, 31\n\t"
+        "v_alignbit_b32 %8, %8, %7, 31\n\t"
+        "v_alignbit_b32 %7, %7, %6, 31\n\t"
+        "v_alignbit_b32 %6, %6, %5, 31\n\t"
+        "v_alignbit_b32 %5, %5, %4, 31\n\t"
+        "v_alignbit_b32 %4, %4, %3, 31\n\t"
+        "v_alignbit_b32 %3, %3, %2, 31\n\t"
+        "v_alignbit_b32 %2, %2, %1, 31\n\t"
+        "v_alignbit_b32 %1, %1, %0, 31\n\t"
+        "v_lshlrev_b32 %0, 1, %0\n\t"
+        "v_add_u32 %11, -1, %11\n\t"
+        "s_mov_b64 exec, %12"
+        : "+&v"(H[0]), "+&v"(H[1]), "+&v"(H[2]), "+&v"(H[3]), "+&v"(H[4]), "+&v"(H[5]), "+&v"(H[6]), "+&v"(H[7]), "+&v"(H[8]), "+&v"(H[9]), "+&v"(H[10]),
           "+&v"(e), "=&s"(sv)
         :
         : "vcc");

@@ -113,7 +113,8 @@ int main(int argc, char** argv)
     state = argc > 1 ? strtoull(argv[1], 0, 10) : 1;
     const long cases = argc > 2 ? atol(argv[2]) : 20000;
     const long bad = all<1>(cases) + all<2>(cases) + all<3>(cases) + all<4>(cases) +
-                     all<5>(cases) + all<6>(cases) + all<7>(cases) + all<8>(cases);
+                     all<5>(cases) + all<6>(cases) + all<7>(cases) + all<8>(cases) +
+                     run<10, true>(0, 4 * cases);
     printf("%ld mismatches\n", bad);
     return bad != 0;
 }

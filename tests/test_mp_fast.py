@@ -1,4 +1,4 @@
-"""The branch-light iteration of up to 8 words (mdz_amd/csrc/mp_fast.h): on
+"""The branch-light iteration of up to 8 words and of 10 whole ones (mdz_amd/csrc/mp_fast.h): on
 the CPU against mp_rn.h, on the GPU against the oracle.  Tolerance: none."""
 import os
 import subprocess
