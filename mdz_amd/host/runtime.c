@@ -348,7 +348,9 @@ static void job_free_mem(mdzg_job* j)
     free(j);
 }
 
-/* about the cycles of one iteration of a wave alone on its SIMD */
+/* about the cycles of one iteration of a wave alone on its SIMD: the loops
+   with few votes (mp_fast.h: up to 8 words and 10 whole ones, an even id), the
+   others */
 static double iteration_cycles(int kid)
 {
     const int nw = mdzg_kid_words(kid);
@@ -356,7 +358,7 @@ static double iteration_cycles(int kid)
         return 60.0;
     if (nw == 0)                 /* GMP: by the bucket's limbs */
         return 1800.0 * mdzg_gmp_limbs[kid - MDZG_KID_GMP0];
-    return nw <= 8 ? 600.0 + 270.0 * nw : 500.0 * nw;
+    return nw <= 8 || (nw == 10 && kid % 2 == 0) ? 600.0 + 270.0 * nw : 500.0 * nw;
 }
 
 static int mdzg_job_start(mdzg_ctx* c, const mdzg_tile* tiles, int ntiles, int mode,
@@ -401,8 +403,8 @@ static int mdzg_job_start(mdzg_ctx* c, const mdzg_tile* tiles, int ntiles, int m
 
     /* Tiles by kernel class (stable).  A batch whose classes leave SIMDs idle
        launches the class whose pixels can take longest first, and classes of
-       few pixels with four lanes each (mdzg_dev_quad_pays): the device runs four queues, and of more classes than that the later ones
-       wait.  Other batches go in the order of kernel ids, the wide classes
+       few pixels with four lanes each (mdzg_dev_quad_pays): the device runs
+       four queues, and of more classes than that the later ones wait.  Other batches go in the order of kernel ids, the wide classes
        last: started first, they share their SIMDs with everything else and
        end later.  The tiles of 12 classes, 1024-bit ones of 3600 iterations
        among them: 24 tiles 15.8 ms with order and four lanes, 20.5 with four
