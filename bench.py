@@ -13,7 +13,10 @@ config 5 rows) and, with --config 3/4/5/gmp, the batched and serving forms,
 the full deep render and the GMP path.
 
 pixel-iterations = sum over samples of (count if count > 0 else depth): the
-iterations the reference loop executes.  Algorithmic operations per
+iterations the reference loop executes.  The kernels end a pixel whose orbit
+is periodic bit for bit (its count is 0 however long it runs), so on views
+with such orbits (config 1, the interior frame) the rates are work rates of
+the reference's iterations, not iterations run.  Algorithmic operations per
 pixel-iteration: 7 FP64 operations (double path), 2n^2+n 32x32-bit
 multiply-accumulates with n = p/32 (RN paths).  The roofline peak is MI355X's
 78.6 TFLOP/s FP64 vector rate; a 32x32->64 multiply-accumulate
@@ -514,10 +517,12 @@ def config5_deep(ctx, M, WL, np, cpu=True):
 
 
 def fp64_interior(ctx, WL, reps=5):
-    """The FP64 kernel on a frame whose pixels all run to depth (1920x1080,
-    depth 2000, 4.15e9 pixel-iterations): the iteration rate without refills.
-    Its loop issues FP64_VALU_PER_ITER VALU instructions per wave-iteration,
-    which bounds the rate at PEAK_VALU_ISSUE * 64 / FP64_VALU_PER_ITER."""
+    """The FP64 kernel on a frame without escapes (1920x1080, depth 2000,
+    4.15e9 pixel-iterations of the reference).  Its loop issues
+    FP64_VALU_PER_ITER VALU instructions per wave-iteration, which bounds the
+    iterations run at PEAK_VALU_ISSUE * 64 / FP64_VALU_PER_ITER a second; the
+    orbits converge to a fixed point and end when they repeat bit for bit, so
+    the rate lies above that bound and has no fraction of a peak."""
     v = WL.interior_view()
     ctx.render(v)
     ks = []
@@ -529,8 +534,9 @@ def fp64_interior(ctx, WL, reps=5):
     bound = PEAK_VALU_ISSUE * 64 / FP64_VALU_PER_ITER
     return dict(workload="1920x1080 inside the main cardioid (-0.1 + 0.1i, width 1e-6), depth 2000",
                 pixel_iters=st["pixel_iters"], kernel_ms=k, kernel_gpix_per_s=rate / 1e9,
-                frac_fp64_peak=7 * rate / 1e12 / PEAK_TOPS,
-                valu_bound_gpix_per_s=bound / 1e9, frac_valu_bound=rate / bound)
+                valu_bound_gpix_per_s=bound / 1e9,
+                note="work rate: orbits that repeat bit for bit end before the depth, so fewer "
+                     "iterations run than pixel_iters counts")
 
 
 FRAC_1024_BASIS = ("algorithmic 2080 32x32-bit MACs (x2 ops) per pixel-iteration: one 32-word "
@@ -771,14 +777,14 @@ def main():
         unl_pr = unloaded_latency(ctx, M, np, M.SERVE_PER_REQUEST, tiles)
         sat_pr = saturation_run(ctx, M, np, M.SERVE_PER_REQUEST, tiles)
         loads = []
-        for f in (0.5, 0.6, 0.7, 0.8, 0.9):
+        for f in (0.4, 0.5, 0.6, 0.7, 0.8, 0.9):
             r = serve_run(ctx, M, np, M.SERVE_BATCHED, tiles, f * sat["tiles_per_s"])
             loads.append(dict(load=f, rate=r["rate"], p50_ms=r["p50_ms"], p99_ms=r["p99_ms"],
                               tiles_per_s=r["tiles_per_s"], gpix_per_s=r["gpix_per_s"],
                               p99_over_unloaded=r["p99_ms"] / unl))
         ok = [x for x in loads if x["p99_over_unloaded"] <= 2.0]
         best = max(ok, key=lambda x: x["gpix_per_s"]) if ok else None
-        half = loads[0]
+        half = loads[1]
         res["latency"] = dict(workload="Poisson requests of 64x64 crops of config 2 (p=128, "
                               "depth 5000), continuous batching", unloaded_p50_ms=unl,
                               saturation_tiles_per_s=sat["tiles_per_s"],
