@@ -215,7 +215,7 @@ __device__ __forceinline__ void quad_run(quad_state<N>& s, const quad_role& r, c
         /* q2: RN(wim2 + wre2) > 4, as escaped_fast (p >= 257 here) */
         const uint32_t ti = qperm<1, 1, 1, 1>(s.p.m[N - 1]);
         const int32_t ei = (int32_t)qperm<1, 1, 1, 1>((uint32_t)s.p.e);
-        const int32_t er = s.p.e;   /* c = 0: exponents down to INT_MIN */
+        const int32_t er = s.p.e;
         const int32_t ai = 5 - (ei < -64 ? -64 : ei), ar = 5 - (er < -64 ? -64 : er);
         const uint32_t si = (uint32_t)(ai < 1 ? 1 : (ai > 31 ? 31 : ai));
         const uint32_t sr = (uint32_t)(ar < 1 ? 1 : (ar > 31 ? 31 : ar));

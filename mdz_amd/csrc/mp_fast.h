@@ -715,9 +715,10 @@ struct rn_form {
     uint32_t va;                  /* 1: hybrid                                */
 };
 
-/* an operand as loaded: a zero's exponent raised to EZF.  A sum with a zero c
-   (a Julia set of c = 0) then flushes values below 2^EZF, whose squares'
-   exponents would otherwise pass the end of an int32 after 30 iterations. */
+/* an operand as loaded: a zero's exponent raised to EZF.  In a sum with a zero
+   c (a Julia set of c = 0) values below 2^EZF then become 0 or, in add_rn, at
+   most a unit of the guard word below 2^EZF; their squares' exponents would
+   otherwise pass the end of an int32 after 30 iterations. */
 template <int N>
 MP_HD void clamp_zero(mp<N>& v)
 {

@@ -48,7 +48,10 @@
 
 namespace mdzg {
 
-static constexpr int32_t EZERO = -(1 << 30);
+/* below every exponent that the loop computes (the squares of values of 2^EZF,
+   mp_fast.h), and high enough that the exponent of a product of two zeros,
+   less its normalising shift, is an int32 */
+static constexpr int32_t EZERO = -(3 << 28);
 
 template <int N>
 struct mp {
@@ -1161,7 +1164,9 @@ MP_HD void add_rn(mp<N>& r, const mp<N>& a_in, const mp<N>& b_in, uint32_t flipb
         e += rs ? 1 : 0;
     }
 
-    /* a borrow (only possible when d == 0, so S == 0): negate, flip sign */
+    /* a borrow (d == 0, so S == 0; or A is a zero c, raised to EZF at load, and
+       B below it: one unit of the guard word is left, a value as small as
+       the zero's exponent): negate, flip sign */
     uint32_t sres = sa;
     /* 0/1 from the data (c is the carry out, 0 or 1), used as a number */
     const uint32_t ngv = (SUBNN ? 1u : sub) & (c ^ 1u);
