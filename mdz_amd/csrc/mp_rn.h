@@ -50,8 +50,10 @@ namespace mdzg {
 
 /* below every exponent that the loop computes (the squares of values of 2^EZF,
    mp_fast.h), and high enough that the exponent of a product of two zeros,
-   less its normalising shift, is an int32 */
-static constexpr int32_t EZERO = -(3 << 28);
+   less its normalising shift, is an int32.  0xc0800000, the bits of -4.0f, is
+   an inline constant of the instructions that select it: with another value
+   the 1024-bit loop holds it in a register and spills 20 bytes a lane more. */
+static constexpr int32_t EZERO = -(1 << 30) + (1 << 23);
 
 template <int N>
 struct mp {
