@@ -108,15 +108,12 @@ __device__ __forceinline__ quad_role quad_role_of()
 template <int N>
 __device__ __forceinline__ void quad_products(quad_state<N>& s, const quad_role& r, int kclr)
 {
-    constexpr int K = limb_count<N>(), L0 = limb_l0<N>(), K0 = L0 - 1;
-    constexpr int TOP = (64 * N + LB - 1) / LB;
-    constexpr int W = LB + limb_s0<N>();
     limb_value<N> x, y;
     {
         limb_value<N> z;
         to_limbs<N>(z, s.v);
 #pragma unroll
-        for (int i = 0; i < K; ++i) {
+        for (int i = 0; i < limb_count<N>(); ++i) {
             x.m.l[i] = qperm<2, 0, 2, 0>(z.m.l[i]);
             y.m.l[i] = qperm<0, 0, 2, 2>(z.m.l[i]);
         }
@@ -127,51 +124,10 @@ __device__ __forceinline__ void quad_products(quad_state<N>& s, const quad_role&
     }
     uint32_t H[N + 1];
     uint64_t low = 0;
-    {
-        uint32_t R[TOP - L0];
-        uint64_t acc = 0;
-#pragma unroll
-        for (int k = K0; k < TOP; ++k) {
-            const int i0 = k < K ? 0 : k - K + 1;
-            if ((k & 1) == 0 && k / 2 < K)
-                acc += (uint64_t)x.m.l[k / 2] * (y.m.l[k / 2] & r.diag);
-            if (2 * i0 < k) {
-                uint64_t o = 0;
-#pragma unroll
-                for (int i = i0; 2 * i < k; ++i)
-                    o += (uint64_t)(i == i0 ? after(x.m.l[i], acc) : x.m.l[i]) * y.m.l[k - i];
-                acc += o << r.dbl;
-            }
-            if (k >= L0)
-                R[k - L0] = (uint32_t)acc & LMASK;
-            else
-                low = (uint32_t)acc & LMASK;
-            acc >>= LB;
-        }
-        low |= (uint64_t)(R[0] & ((1u << limb_s0<N>()) - 1u)) << LB;
-        from_limbs<N + 1, N - 1, L0, TOP - L0>(H, R);
-    }
+    half_mul<N>(x.m, y.m, r.dbl, r.diag, H, low);
     /* q0: its half and q3's */
-    low += (uint64_t)(qperm<3, 3, 3, 3>((uint32_t)low) & r.join) |
-           (uint64_t)(qperm<3, 3, 3, 3>((uint32_t)(low >> 32)) & r.join) << 32;
-    uint32_t c = (uint32_t)(low >> W);
-    low &= ((uint64_t)1 << W) - 1u;
-#pragma unroll
-    for (int j = 0; j <= N; ++j) H[j] = add_cc(H[j], qperm<3, 3, 3, 3>(H[j]) & r.join, c, c);
-    const int32_t e0 = x.e + y.e;
-    int32_t e = e0;
-    uint32_t S = 1;
-    norm_product<N>(H, e);
-    if (__builtin_expect(wave_any(short_unsure<N>(H[0], kclr) & (r.diag != 0)), 0)) {
-        const uint32_t un = (uint32_t)(e0 - e);
-#pragma unroll
-        for (int j = 0; j < N; ++j) H[j] = un ? funnel_r(H[j + 1], H[j], 1u) : H[j];
-        H[N] >>= un;
-        limb_rest<N, false>(x.m, y.m, H, low, S);
-        e = e0;
-        norm_product<N>(H, e);
-    }
-    round_product<N>(s.p, H, S, e, x.s ^ y.s, kclr);
+    half_join<N>(H, low, [&](uint32_t v, int) { return qperm<3, 3, 3, 3>(v) & r.join; });
+    half_round<N>(s.p, x, y, H, low, r.diag, kclr);
 }
 
 /* Up to n passes of the quads of live, fewer once none is left: the sums

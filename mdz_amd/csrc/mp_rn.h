@@ -875,9 +875,18 @@ MP_HD void limb_col(const limbs<N>& a, const limbs<N>& b, int k, uint64_t& acc)
     }
 }
 
-/* limb of the guard word's lowest bit, and that bit's place in it */
+/* limb of the guard word's lowest bit (K0 = l0 - 1 is the lowest column
+   formed), and that bit's place in it.  Checked for whoever forms such a
+   product: a column's products fit the accumulator, and the columns left out
+   stay below the guard word (equal at 12 words: 352 bits). */
 template <int N>
-constexpr int limb_l0() { return 32 * (N - 1) / LB; }
+constexpr int limb_l0()
+{
+    constexpr int L0 = 32 * (N - 1) / LB;
+    static_assert(limb_count<N>() <= 38 && LB * L0 + stages(L0 - 1) <= 32 * (N - 1),
+                  "bounds above");
+    return L0;
+}
 template <int N>
 constexpr int limb_s0() { return 32 * (N - 1) % LB; }
 
@@ -888,8 +897,6 @@ MP_HD void limb_mul(const limbs<N>& a, const limbs<N>& b, uint32_t* H, uint64_t&
 {
     constexpr int L0 = limb_l0<N>(), K0 = L0 - 1;
     constexpr int TOP = (64 * N + LB - 1) / LB;   /* limbs of the whole product */
-    static_assert(limb_count<N>() <= 38 && LB * (K0 + 1) + stages(K0) <= 32 * (N - 1),
-                  "bounds above");
     uint32_t R[TOP - L0];
     uint64_t acc = 0;
 #pragma unroll
@@ -1013,6 +1020,76 @@ MP_HD void mul_limbs(mp<N>& r, const limb_value<N>& a, const limb_value<N>& b, i
         norm_product<N>(H, e);
     }
     round_product<N>(r, H, S, e, SQR ? 0u : (a.s ^ b.s), kclr);
+}
+
+/* The product of k_quad.h, in two halves: the columns k >= K0 of the sum of
+   x[i] y[k-i] over i < k-i, shifted by dbl, with the diagonal where diag is
+   all ones.  x * y is the half (x, y, 0, ~0) and the half (y, x, 0, 0); x * x
+   is (x, x, 1, ~0) alone.  H and low as in limb_mul. */
+template <int N>
+MP_HD void half_mul(const limbs<N>& x, const limbs<N>& y, uint32_t dbl, uint32_t diag, uint32_t* H,
+                    uint64_t& low)
+{
+    constexpr int K = limb_count<N>(), L0 = limb_l0<N>(), K0 = L0 - 1;
+    constexpr int TOP = (64 * N + LB - 1) / LB;
+    uint32_t R[TOP - L0];
+    uint64_t acc = 0;
+#pragma unroll
+    for (int k = K0; k < TOP; ++k) {
+        const int i0 = k < K ? 0 : k - K + 1;
+        if ((k & 1) == 0 && k / 2 < K)
+            acc += (uint64_t)x.l[k / 2] * (y.l[k / 2] & diag);
+        if (2 * i0 < k) {
+            uint64_t o = 0;
+#pragma unroll
+            for (int i = i0; 2 * i < k; ++i)
+                o += (uint64_t)(i == i0 ? after(x.l[i], acc) : x.l[i]) * y.l[k - i];
+            acc += o << dbl;
+        }
+        if (k >= L0)
+            R[k - L0] = (uint32_t)acc & LMASK;
+        else
+            low = (uint32_t)acc & LMASK;
+        acc >>= LB;
+    }
+    low |= (uint64_t)(R[0] & ((1u << limb_s0<N>()) - 1u)) << LB;
+    from_limbs<N + 1, N - 1, L0, TOP - L0>(H, R);
+}
+
+/* H and low += the other half's, of which other(v, j) is word j for a word v
+   of this one: -2 and -1 the words of low, then H */
+template <int N, class OTHER>
+MP_HD void half_join(uint32_t* H, uint64_t& low, OTHER other)
+{
+    constexpr int W = LB + limb_s0<N>();
+    low += (uint64_t)other((uint32_t)low, -2) | (uint64_t)other((uint32_t)(low >> 32), -1) << 32;
+    uint32_t c = (uint32_t)(low >> W);
+    low &= ((uint64_t)1 << W) - 1u;
+#pragma unroll
+    for (int j = 0; j <= N; ++j) H[j] = add_cc(H[j], other(H[j], j), c, c);
+}
+
+/* r = the rounded product of x and y from its joined H and low; want: all ones
+   where it is needed */
+template <int N>
+MP_HD void half_round(mp<N>& r, const limb_value<N>& x, const limb_value<N>& y, uint32_t* H,
+                      uint64_t low, uint32_t want, int kclr)
+{
+    const int32_t e0 = x.e + y.e;
+    int32_t e = e0;
+    uint32_t S = 1;
+    norm_product<N>(H, e);
+    if (__builtin_expect(wave_any(short_unsure<N>(H[0], kclr) & (want != 0)), 0)) {
+        MDZG_NOTE_SHORT_FALLBACK();
+        const uint32_t un = (uint32_t)(e0 - e);
+#pragma unroll
+        for (int j = 0; j < N; ++j) H[j] = un ? funnel_r(H[j + 1], H[j], 1u) : H[j];
+        H[N] >>= un;
+        limb_rest<N, false>(x.m, y.m, H, low, S);
+        e = e0;
+        norm_product<N>(H, e);
+    }
+    round_product<N>(r, H, S, e, x.s ^ y.s, kclr);
 }
 
 /* r = RN_p(a * b) (SQR: b ignored, a*a) */
