@@ -850,6 +850,7 @@ __device__ constexpr bool rn_lazy() { return FULL && N >= 12; }
 template <int N, bool FULL, bool LAZY = false>
 __device__ __forceinline__ bool rn_step(rn_state<N>& s, int fractal, int32_t wz, int kclr)
 {
+    static_assert(!rn_fast<N, FULL>(), "these word counts iterate by step_fast");
     const int k = FULL ? 0 : kclr;
     constexpr bool LZ = LAZY && rn_lazy<N, FULL>();
     constexpr int32_t GAP = 32 * N + 2;
@@ -1016,21 +1017,200 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_tile(cons
     t.out[idx] = count;
 }
 
-/* Per-operation probe (measurement only, p = 32N).  Each lane takes its
-   pixel of the tile, runs `warm` iterations of the escape loop so that its
-   values carry the orbit's exponents and bit patterns (lanes of a wave
-   neighbours, as in a render), then repeats one operation `reps` times in a
-   dependent chain whose operands keep those statistics:
+/* Per-operation probe (measurement only, p = 32N): the operations and the
+   iteration that the render kernels of N words run.  Each lane takes its pixel
+   of the tile, runs `warm` iterations of the escape loop so that its values
+   carry the orbit's exponents and bit patterns (lanes of a wave neighbours, as
+   in a render), then repeats one operation `reps` times in a dependent chain
+   whose operands keep those statistics:
      MDZG_OPP_LOOP   the loop alone (the chain's register dependency only)
-     MDZG_OPP_MUL    x = RN(x * y)
-     MDZG_OPP_SQR    x = RN(x^2) with the exponent set back to 0
+     MDZG_OPP_MUL    x = RN(x * y); in limbs, the product of z's
+     MDZG_OPP_SQR    x = RN(x^2) with the exponent set back to 0; in limbs, the
+                     square of z's real part
      MDZG_OPP_ADD    x = RN(x + c_re), then x = RN(x - c_re): two a rep
      MDZG_OPP_SUBNN  a = |RN(a - b)|, a and b the squares (the SUB_NONNEG form)
      MDZG_OPP_ESC    the escape test on the squares
      MDZG_OPP_STEP   the whole iteration
+   The operations of mp_fast.h leave their rare lanes to a vote that the
+   iteration takes once for several: here each has its own.  The limbs of z are
+   formed once an iteration, so the products in limbs take them as they are
+   and only the iteration holds the conversion.
    Counter passes over the launches give each operation's instructions.  A
    word of the result goes to the tile's output so that nothing is removed;
    it is not a count. */
+template <int N>
+__device__ __forceinline__ uint32_t rn_op_fast(rn_state<N>& s, mp<N>& x, int op, int fractal,
+                                               int warm, int reps)
+{
+    const lanes all = scalar_copy(lanes_of(true));
+    const rn_prec<true> pr;
+    const rn_form fm = form_of(fractal);
+    lanes live = all, rare = 0;
+    int32_t wz = 0;
+    rn_run<N, true>(s, fm, pr, wz, live, warm);
+    x = s.wre;
+    uint32_t h = 0;
+    const mp<N> y = s.wim, cr = s.c.get_re(), ci = s.c.get_im();
+    switch (op) {
+    case MDZG_OPP_MUL:
+        for (int i = 0; i < reps; ++i) {
+            mp<N> z;
+            rare = 0;
+            mul_fast<N, true, false>(z, x, y, pr, rare);
+            if (__builtin_expect((rare & all) != 0, 0))
+                mul_rn<N, false>(z, x, y, 0);
+            x = z;
+        }
+        break;
+    case MDZG_OPP_SQR:
+        for (int i = 0; i < reps; ++i) {
+            mp<N> z;
+            rare = 0;
+            mul_fast<N, true, true>(z, x, x, pr, rare);
+            if (__builtin_expect((rare & all) != 0, 0))
+                mul_rn<N, true>(z, x, x, 0);
+            x = z;
+            x.e = 0;
+        }
+        break;
+    case MDZG_OPP_ADD:
+        for (int i = 0; i < 2 * reps; ++i) {
+            mp<N> z;
+            aligned<N> a;
+            uint32_t S = 0;
+            rare = 0;
+            align_fast<N>(a, x, cr);
+            if ((lanes_of(is_far<N>(a)) & all) != 0)
+                align_far<N>(a, S, all);
+            sum_fast<N, true, false>(z, a, x.s, cr.s ^ ((uint32_t)i & 1u), S, pr, rare);
+            if (__builtin_expect((rare & all) != 0, 0)) {
+                add_rn<N>(z, x, cr, (uint32_t)i & 1u, 0);
+                clamp_zero<N>(z);
+            }
+            x = z;
+        }
+        break;
+    case MDZG_OPP_SUBNN:
+        for (int i = 0; i < reps; ++i) {
+            mp<N> z;
+            aligned<N> a;
+            uint32_t S = 0;
+            rare = 0;
+            align_fast<N>(a, s.wre2, s.wim2);
+            if ((lanes_of(is_far<N>(a)) & all) != 0)
+                align_far<N>(a, S, all);
+            sum_fast<N, true, true>(z, a, 0u, 1u, S, pr, rare);
+            if (__builtin_expect((rare & all) != 0, 0)) {
+                add_rn<N, SUB_NONNEG>(z, s.wre2, s.wim2, 1u, 0);
+                clamp_zero<N>(z);
+            }
+            z.s = 0;
+            s.wre2 = z;
+        }
+        break;
+    case MDZG_OPP_ESC:
+        for (int i = 0; i < reps; ++i) {
+            rare = 0;
+            h += (uint32_t)escaped_fast<N, true>(s.wim2, s.wre2, pr, rare) + (uint32_t)rare;
+            asm volatile("" : "+v"(s.wim2.m[N - 1]));
+        }
+        break;
+    case MDZG_OPP_STEP:
+        for (int i = 0; i < reps; ++i)
+            h += (uint32_t)step_fast<N, true>(s.wre, s.wim, s.wre2, s.wim2, cr, ci, fm, pr, i,
+                                              live);
+        break;
+    default:
+        for (int i = 0; i < reps; ++i)
+            asm volatile("" : "+v"(x.m[0]));
+        break;
+    }
+    return h;
+}
+
+/* x is used and z is another one, as far as the compiler knows: nothing of a
+   product of z is moved out of the loop or left out */
+template <int N>
+__device__ __forceinline__ void renew(rn_state<N>& s, const mp<N>& x)
+{
+    asm volatile("" ::"v"(x.e));
+#pragma unroll
+    for (int j = 0; j < N; ++j) asm volatile("" ::"v"(x.m[j]));
+#pragma unroll
+    for (int i = 0; i < limb_count<N>(); ++i)
+        asm volatile("" : "+v"(s.lre.m.l[i]), "+v"(s.lim.m.l[i]));
+}
+
+template <int N>
+__device__ __forceinline__ uint32_t rn_op_wide(rn_state<N>& s, mp<N>& x, int op, int fractal,
+                                               int warm, int reps)
+{
+    for (int32_t wz = 1; wz <= warm; ++wz)
+        (void)rn_step<N, true, true>(s, fractal, wz, 0);
+    if (s.lazy)
+        sqr_im<N>(s.wim2, s, 0);
+    s.lazy = false;
+    rn_words<N>(s);
+    x = s.wre;
+    const mp<N> y = s.wim;
+    const double thresh = 4.0 + ldexp(1.0, 2 - 32 * N);
+    uint32_t h = 0;
+    /* one loop per operation, so that no loop carries the other
+       operations' values */
+    switch (op) {
+    case MDZG_OPP_MUL:
+        for (int i = 0; i < reps; ++i) {
+            if constexpr (limb_product<N>()) {
+                mul_re_im<N>(x, s, 0);
+                renew<N>(s, x);
+            } else {
+                mul_rn<N, false>(x, x, y, 0);
+            }
+        }
+        break;
+    case MDZG_OPP_SQR:
+        for (int i = 0; i < reps; ++i) {
+            if constexpr (limb_product<N>()) {
+                sqr_re<N>(x, s, 0);
+                renew<N>(s, x);
+            } else {
+                mul_rn<N, true>(x, x, x, 0);
+                x.e = is_zero(x) ? x.e : 0;
+            }
+        }
+        break;
+    case MDZG_OPP_ADD:
+        for (int i = 0; i < reps; ++i) {
+            add_rn<N>(x, x, s.c.get_re(), 0u, 0);
+            add_rn<N>(x, x, s.c.get_re(), 1u, 0);
+        }
+        break;
+    case MDZG_OPP_SUBNN:
+        for (int i = 0; i < reps; ++i) {
+            add_rn<N, SUB_NONNEG, true>(x, s.wre2, s.wim2, 1u, 0);
+            x.s = 0;
+            s.wre2 = x;
+        }
+        break;
+    case MDZG_OPP_ESC:
+        for (int i = 0; i < reps; ++i) {
+            h += escaped<N>(s.wim2, s.wre2, thresh, 0) ? 1u : 0u;
+            asm volatile("" : "+v"(s.wim2.m[0]));
+        }
+        break;
+    case MDZG_OPP_STEP:
+        for (int i = 0; i < reps; ++i)
+            h += rn_step<N, true, true>(s, fractal, i, 0) ? 1u : 0u;
+        rn_words<N>(s);
+        break;
+    default:
+        for (int i = 0; i < reps; ++i)
+            asm volatile("" : "+v"(x.m[0]));
+        break;
+    }
+    return h;
+}
+
 template <int N>
 __global__ __launch_bounds__(256, (rn_min_waves<N, true>())) void k_rn_op_probe(
     const mdzg_dtile* tp, int op, int warm, int reps)
@@ -1045,55 +1225,12 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, true>())) void k_rn_op_probe(
     rn_state<N> s;
     s.c.init(c_lds);
     rn_init<N, true>(s, t, row, col);
-    const int fractal = t.fractal;
-    for (int32_t wz = 1; wz <= warm; ++wz)
-        (void)rn_step<N, true>(s, fractal, wz, 0);
-    rn_words<N>(s);
-    const double thresh = 4.0 + ldexp(1.0, 2 - 32 * N);
-    uint32_t h = 0;
-    mp<N> x = s.wre, y = s.wim;
-    /* one loop per operation, so that no loop carries the other
-       operations' values */
-    switch (op) {
-    case MDZG_OPP_MUL:
-        for (int i = 0; i < reps; ++i)
-            mul_rn<N, false>(x, x, y, 0);
-        break;
-    case MDZG_OPP_SQR:
-        for (int i = 0; i < reps; ++i) {
-            mul_rn<N, true>(x, x, x, 0);
-            x.e = is_zero(x) ? x.e : 0;
-        }
-        break;
-    case MDZG_OPP_ADD:
-        for (int i = 0; i < reps; ++i) {
-            add_rn<N>(x, x, s.c.get_re(), 0u, 0);
-            add_rn<N>(x, x, s.c.get_re(), 1u, 0);
-        }
-        break;
-    case MDZG_OPP_SUBNN:
-        for (int i = 0; i < reps; ++i) {
-            add_rn<N, SUB_NONNEG>(x, s.wre2, s.wim2, 1u, 0);
-            x.s = 0;
-            s.wre2 = x;
-        }
-        break;
-    case MDZG_OPP_ESC:
-        for (int i = 0; i < reps; ++i) {
-            h += escaped<N>(s.wim2, s.wre2, thresh, 0) ? 1u : 0u;
-            asm volatile("" : "+v"(s.wim2.m[0]));
-        }
-        break;
-    case MDZG_OPP_STEP:
-        for (int i = 0; i < reps; ++i)
-            h += rn_step<N, true>(s, fractal, i, 0) ? 1u : 0u;
-        break;
-    default:
-        for (int i = 0; i < reps; ++i)
-            asm volatile("" : "+v"(x.m[0]));
-        break;
-    }
-    rn_words<N>(s);
+    mp<N> x;
+    uint32_t h;
+    if constexpr (rn_fast<N, true>())
+        h = rn_op_fast<N>(s, x, op, t.fractal, warm, reps);
+    else
+        h = rn_op_wide<N>(s, x, op, t.fractal, warm, reps);
     t.out[idx] = h ^ x.m[N - 1] ^ s.wre.m[N - 1] ^ s.wre2.m[N - 1];
 }
 
