@@ -180,6 +180,19 @@ int mdzg_dev_quad_pays(int kid, uint64_t total, int ncu)
     return f != nullptr;
 }
 
+/* dynamic LDS with which a persistent launch's blocks take more than half of a
+   CU's 160 KB each */
+unsigned mdzg_dev_spread(int kid)
+{
+    const void* f;
+    lookup(kid, 1, &f);
+    hipFuncAttributes a;
+    if (!f || hipFuncGetAttributes(&a, f) != hipSuccess)
+        return 0;
+    const size_t want = (size_t)81 << 10;
+    return a.sharedSizeBytes < want ? (unsigned)(want - a.sharedSizeBytes) : 0u;
+}
+
 /* blocks of a persistent (slice) launch: one lane a pixel, four with quad,
    at most blocks_per_cu a CU */
 int mdzg_dev_grid(uint64_t total, int quad, int ncu, int blocks_per_cu)

@@ -21,6 +21,7 @@ int mdzg_dev_nkernels(void);
    where the kernel has no such form) */
 int mdzg_dev_occupancy(int kid, int form);
 int mdzg_dev_quad_pays(int kid, uint64_t total, int ncu);
+unsigned mdzg_dev_spread(int kid);
 int mdzg_dev_grid(uint64_t total, int quad, int ncu, int blocks_per_cu);
 int mdzg_dev_launch_tile(int kid, const mdzg_dtile* d_tile, uint32_t npix, hipStream_t st);
 int mdzg_dev_launch_persist(int kid, const mdzg_dtile* d_tiles, int ntiles, uint64_t total,
@@ -77,6 +78,15 @@ int mdzg_rt_submit_image(mdzg_ctx* c, const mdzg_tile* tile, const mdzg_image_re
 /* validation shared by the colouring entry points */
 int mdzg_palette_ok(const mdzg_palette* p);
 
+/* a tile of a batch, for its launch plan (runtime.c) */
+typedef struct mdzg_plan_tile {
+    int kid;
+    long long depth;
+    uint64_t pixels;
+} mdzg_plan_tile;
+enum { MDZG_PLAN_FOUR = 1, MDZG_PLAN_SPREAD = 2 };
+int mdzg_plan_batch(const mdzg_plan_tile* t, int n, int ncu, int* kids, int* how);
+
 int mdzg_kid_words(int kid);   /* words of an RN kernel id, 0 for another */
 extern const int mdzg_gmp_limbs[MDZG_NGMP];
 
@@ -130,6 +140,7 @@ struct mdzg_ctx {
     int* d_cancel_zero;         /* a device int that stays 0 */
     int occ[MDZG_NKERNELS];     /* resident blocks per CU (persistent grid) */
     int occ_quad[MDZG_NKERNELS];   /* the same of the four-lane form, 0: none */
+    unsigned spread[MDZG_NKERNELS];   /* LDS that keeps a second block off the CU */
     int chunk[MDZG_NKERNELS];   /* iterations between lane refills */
     pthread_mutex_t lock;
     /* mdzg_render_tile_noalloc: the device address of the library's static

@@ -22,7 +22,12 @@
 #include "mdzg_host.h"
 
 #define NSTREAMS 8
-#define MOST_IDLE_JOBS 3      /* with more in flight a job takes the chip as busy */
+/* Jobs launched and not yet waited for (finished ones, too, until the program
+   waits) from which on a job takes one lane a pixel: with several of 160x160
+   pixels the chip is busy (eight at 700 bits 44 ms, with four lanes for all 50).
+   Small ones pay for it: eight of 96x96 at 1024 bits take 109 ms, with four
+   lanes for all 62, with one lane for all 128. */
+#define MOST_IDLE_JOBS 3
 #define NCACHE 8
 #define ALIGN_UP(x, a) (((x) + (size_t)(a) - 1) & ~((size_t)(a) - 1))
 
@@ -160,6 +165,7 @@ int mdzg_create(int device, mdzg_ctx** out)
         if (c->occ[k] < 1)
             c->occ[k] = 1;
         c->occ_quad[k] = mdzg_dev_occupancy(k, 3);
+        c->spread[k] = mdzg_dev_spread(k);
         c->chunk[k] = default_chunk(k);
     }
     c->graphs = 1;
@@ -361,6 +367,67 @@ static double iteration_cycles(int kid)
     return nw <= 8 || (nw == 10 && kid % 2 == 0) ? 600.0 + 270.0 * nw : 500.0 * nw;
 }
 
+/* The classes of a batch in the order of their launches, kids[0 .. return), and
+   in *how the flags MDZG_PLAN_*.  Measured on 94 mixes of 1 to 12 classes, 2 to
+   84 tiles and 48x48 to 1024x1024 pixels, by the batch's load: at a wave per
+   SIMD, four-lane classes at twice their one-lane cycles, against its slowest
+   pixel.
+
+   FOUR: classes of few pixels may take four lanes a pixel (mdzg_dev_quad_pays),
+   and the class whose pixels can take longest goes first, while the batch
+   leaves SIMDs idle.  24 tiles of 9 classes, 96x96 pixels at 1024 bits among
+   them, take 15.3 ms, with one lane 21.4; 7 classes of 300 to 1000 bits, 128x128
+   pixels each (load 1.5), 21.9 and 28.4; 14 tiles of 96x96 (1.7) 25.8 and 28.6.
+   The line lies at a load of 1.9, past which four lanes cost up to 1.5 times,
+   and with more classes than two rounds of the device's four queues at 1.45
+   (36 tiles of 9 classes, 1.7: 27 ms with four lanes, 22.8 without).
+
+   SPREAD: past 1.9 the slowest class goes first, too, its blocks no two to a
+   CU while there are CUs for all.  In the order of kernel ids the wide classes
+   start last, on a chip that the others have filled unevenly, two blocks to a
+   CU: 60 tiles of 9 classes 39 ms by ids, 29 so; 14 tiles of 128x128 at 300 to
+   1000 bits 38.7 and 34.  First without the spread, a launch that comes a
+   tenth of a millisecond after the other queues' ends up the same way: 30
+   tiles of 6 classes 22 or 35 ms.
+
+   Between the lines the order of ids is the safer one (36 tiles 22.8 ms,
+   slowest first 22 or 34). */
+int mdzg_plan_batch(const mdzg_plan_tile* t, int n, int ncu, int* kids, int* how)
+{
+    uint64_t pixels[MDZG_NKERNELS] = { 0 };
+    double most[MDZG_NKERNELS] = { 0.0 };
+    double slowest = 0.0, load = 0.0;
+    int nkid = 0;
+    for (int i = 0; i < n; ++i)
+        pixels[t[i].kid] += t[i].pixels;
+    for (int i = 0; i < n; ++i) {
+        const int kid = t[i].kid;
+        const double c = (double)t[i].depth * iteration_cycles(kid);
+        most[kid] = c > most[kid] ? c : most[kid];
+        slowest = c > slowest ? c : slowest;
+        load += (mdzg_dev_quad_pays(kid, pixels[kid], ncu) ? 2.0 : 1.0) * c * (double)t[i].pixels;
+    }
+    int classes = 0;
+    for (int q = 0; q < MDZG_NKERNELS; ++q)
+        classes += pixels[q] != 0;
+    load /= slowest * 256.0 * (double)ncu;
+    /* a class alone has no others to share with */
+    *how = classes == 1 || load <= (classes <= 8 ? 1.9 : 1.45) ? MDZG_PLAN_FOUR
+           : load > 1.9                                         ? MDZG_PLAN_SPREAD
+                                                                : 0;
+    for (;;) {
+        int k = -1;
+        for (int q = 0; q < MDZG_NKERNELS; ++q)
+            if (pixels[q] && (k < 0 || (*how && most[q] > most[k])))
+                k = q;
+        if (k < 0)
+            break;
+        pixels[k] = 0;
+        kids[nkid++] = k;
+    }
+    return nkid;
+}
+
 static int mdzg_job_start(mdzg_ctx* c, const mdzg_tile* tiles, int ntiles, int mode,
                           const mdzg_image_req* img, int sync, mdzg_job** out)
 {
@@ -383,9 +450,11 @@ static int mdzg_job_start(mdzg_ctx* c, const mdzg_tile* tiles, int ntiles, int m
     j->out_off = (size_t*)malloc(sizeof(size_t) * (size_t)ntiles);
     mdzg_pview* pv = (mdzg_pview*)calloc((size_t)ntiles, sizeof(mdzg_pview));
     int* order = (int*)malloc(sizeof(int) * (size_t)ntiles);
-    if (!j->tiles || !j->out_off || !pv || !order) {
+    mdzg_plan_tile* pt = (mdzg_plan_tile*)malloc(sizeof(mdzg_plan_tile) * (size_t)ntiles);
+    if (!j->tiles || !j->out_off || !pv || !order || !pt) {
         free(pv);
         free(order);
+        free(pt);
         job_free_mem(j);
         return MDZG_ERR_NOMEM;
     }
@@ -401,49 +470,21 @@ static int mdzg_job_start(mdzg_ctx* c, const mdzg_tile* tiles, int ntiles, int m
         goto done;
     }
 
-    /* Tiles by kernel class (stable).  A batch whose classes leave SIMDs idle
-       launches the class whose pixels can take longest first, and classes of
-       few pixels with four lanes each (mdzg_dev_quad_pays): the device runs
-       four queues, and of more classes than that the later ones wait.  Other batches go in the order of kernel ids, the wide classes
-       last: started first, they share their SIMDs with everything else and
-       end later.  The tiles of 12 classes, 1024-bit ones of 3600 iterations
-       among them: 24 tiles 15.8 ms with order and four lanes, 20.5 with four
-       lanes alone, 24.4 with neither; 36 tiles 28 ms, 25.9 and 22.7. */
-    int idle = 1;
+    /* tiles by kernel class (stable) */
+    int how = 0, idle = 0;
     {
-        uint64_t pixels[MDZG_NKERNELS] = { 0 };
-        double most[MDZG_NKERNELS] = { 0.0 };
-        double slowest = 0.0, load = 0.0;
-        for (int i = 0; i < ntiles; ++i)
-            pixels[pv[i].kid] += (uint64_t)tiles[i].ncols * (uint64_t)tiles[i].nlines;
         for (int i = 0; i < ntiles; ++i) {
-            const int kid = pv[i].kid;
-            const double t = (double)tiles[i].view.depth * iteration_cycles(kid);
-            most[kid] = t > most[kid] ? t : most[kid];
-            slowest = t > slowest ? t : slowest;
-            load += (mdzg_dev_quad_pays(kid, pixels[kid], c->ncu) ? 2.0 : 1.0) * t *
-                    (double)tiles[i].ncols * (double)tiles[i].nlines;
+            pt[i].kid = pv[i].kid;
+            pt[i].depth = tiles[i].view.depth;
+            pt[i].pixels = (uint64_t)tiles[i].ncols * (uint64_t)tiles[i].nlines;
         }
-        /* the batch at a wave per SIMD, four-lane classes at twice their
-           one-lane cycles, against its slowest pixel: 1.1 times at 24 tiles
-           above, 1.7 at 36.  A class alone has no others to share with. */
-        int nkid = 0;
-        for (int k = 0; k < MDZG_NKERNELS; ++k)
-            nkid += pixels[k] != 0;
-        idle = (nkid == 1 || load <= 1.45 * slowest * 256.0 * (double)c->ncu) &&
-               __atomic_load_n(&c->jobs, __ATOMIC_RELAXED) < MOST_IDLE_JOBS;
+        j->nkid = mdzg_plan_batch(pt, ntiles, c->ncu, j->kids, &how);
+        idle = how == MDZG_PLAN_FOUR && __atomic_load_n(&c->jobs, __ATOMIC_RELAXED) < MOST_IDLE_JOBS;
         int n = 0;
-        while (j->nkid < nkid) {
-            int k = -1;
-            for (int q = 0; q < MDZG_NKERNELS; ++q)
-                if (pixels[q] && (k < 0 || (idle && most[q] > most[k])))
-                    k = q;
-            pixels[k] = 0;
+        for (int k = 0; k < j->nkid; ++k)
             for (int i = 0; i < ntiles; ++i)
-                if (pv[i].kid == k)
+                if (pt[i].kid == j->kids[k])
                     order[n++] = i;
-            j->kids[j->nkid++] = k;
-        }
     }
 
     /* layout */
@@ -595,6 +636,8 @@ static int mdzg_job_start(mdzg_ctx* c, const mdzg_tile* tiles, int ntiles, int m
                     rc = MDZG_ERR_DEVICE;
                     goto done;
                 }
+                if (how == MDZG_PLAN_SPREAD && k == 0 && grid <= c->ncu)
+                    par[npar - 1].shmem = c->spread[kid];
             }
             first += cnt;
         }
@@ -728,6 +771,7 @@ done:
         mdzg_view_clear(&pv[i]);
     free(pv);
     free(order);
+    free(pt);
     if (rc != MDZG_OK) {
         /* nothing the job launched may still use its memory: wait for its
            stream and for the side streams its class launches forked onto */

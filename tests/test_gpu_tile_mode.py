@@ -1,7 +1,7 @@
 """One launch a tile (BATCH_PER_TILE) iterates FP64 pixels as the persistent
 launch does.  The orbits are bounded for their depth and slow to settle, so the
 time is that of the iterations alone; the bound leaves the launches of four
-tiles and the clock room (1.0 when this was written, 1.7 with the loop of a
+tiles and the clock room (1.0 when this was written, 3.6 with the loop of a
 branch a lane)."""
 import numpy as np
 import pytest
