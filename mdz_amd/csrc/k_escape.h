@@ -72,6 +72,19 @@ __device__ __forceinline__ int read_cancel(const volatile int* p)
     return *(g_cflag*)p;
 }
 
+/* Rounds between two reads of the cancel flag, less 1: 15, fewer where the chunk
+   would make them more than MOST iterations, so that a long chunk does not
+   make a cancelled job run on.  512 iterations up to 10 words (0.7 ms at 128
+   bits; a read waits for the count stores before it, and every 128 iterations
+   cost frames of quickly escaping pixels 5 to 15 % at 80 bits), 128 for wider
+   ones (1.2 ms at 512 bits). */
+template <int MOST>
+__device__ __forceinline__ uint32_t cancel_mask(int chunk)
+{
+    /* >=: with <= the compiler holds the steps in vector registers */
+    return chunk >= MOST ? 0u : (chunk >= MOST / 2 ? 1u : (chunk >= MOST / 4 ? 3u : (chunk >= MOST / 8 ? 7u : 15u)));
+}
+
 /* Queue slots are claimed per wave.  A wave whose lanes need n slots takes
    what is left of its run first; the rest comes from one atomic on the
    shared counter, which takes max(missing, RUN) consecutive slots, the
@@ -1286,6 +1299,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
     bool active = false;
     int fractal = 0, kclr = 0;
     uint32_t round = 0;
+    const uint32_t often = cancel_mask<(N < 12 ? 512 : 128)>(chunk);
     int32_t wz = 0, depth = 0;
     uint32_t* out = nullptr;
     __shared__ uint32_t c_lds[c_in_lds<N>() ? 2 * (N + 2) * 256 : 1];
@@ -1338,7 +1352,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
         }
         if (!__any(active))
             break;
-        const int stop = ((++round & 15) == 0) ? read_cancel(cancel) : 0;
+        const int stop = ((++round & often) == 0) ? read_cancel(cancel) : 0;
         if constexpr (rn_fast<N, FULL>()) {
             /* no active lane reaches its depth within rem iterations: lanes
                that finish leave it a bound, a refill (rem = 0) does not */

@@ -225,6 +225,7 @@ __global__ __launch_bounds__(256, 2) void k_rn_quad(const mdzg_dtile* tiles, int
     bool active = false, drained = false;
     int kclr = 0;
     uint32_t round = 0;
+    const uint32_t often = cancel_mask<128>(chunk);
     int32_t wz = 0, depth = 0;
     uint32_t* out = nullptr;
     rn_form fm = { 1u, 1u, 0u };
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(256, 2) void k_rn_quad(const mdzg_dtile* tiles, int
         }
         if (!__any(active))
             break;
-        const int stop = ((++round & 15) == 0) ? read_cancel(cancel) : 0;
+        const int stop = ((++round & often) == 0) ? read_cancel(cancel) : 0;
         /* passes that no lane's depth ends; a fresh pixel's first makes no
            iteration */
         const int todo = depth - wz < chunk ? depth - wz : chunk;
