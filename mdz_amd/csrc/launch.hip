@@ -29,14 +29,6 @@ void mdzg_kget_rn20(int, const void**, const void**, const void**);
 void mdzg_kget_rn24(int, const void**, const void**, const void**);
 void mdzg_kget_rn28(int, const void**, const void**, const void**);
 void mdzg_kget_rn32(int, const void**, const void**, const void**);
-void mdzg_kquad_rn1(int, const void**, const void**);
-void mdzg_kquad_rn2(int, const void**, const void**);
-void mdzg_kquad_rn3(int, const void**, const void**);
-void mdzg_kquad_rn4(int, const void**, const void**);
-void mdzg_kquad_rn5(int, const void**, const void**);
-void mdzg_kquad_rn6(int, const void**, const void**);
-void mdzg_kquad_rn7(int, const void**, const void**);
-void mdzg_kquad_rn8(int, const void**, const void**);
 void mdzg_kquad_rn10(int, const void**, const void**);
 void mdzg_kquad_rn12(int, const void**, const void**);
 void mdzg_kquad_rn14(int, const void**, const void**);
@@ -59,8 +51,8 @@ static const kget_fn kget_rn[MDZG_NCLASS_N] = {
 };
 typedef void (*kquad_fn)(int, const void**, const void**);
 static const kquad_fn kquad_rn[MDZG_NCLASS_N] = {
-    mdzg_kquad_rn1,  mdzg_kquad_rn2,  mdzg_kquad_rn3,  mdzg_kquad_rn4,
-    mdzg_kquad_rn5,  mdzg_kquad_rn6,  mdzg_kquad_rn7,  mdzg_kquad_rn8,
+    nullptr,         nullptr,         nullptr,         nullptr,
+    nullptr,         nullptr,         nullptr,         nullptr,
     mdzg_kquad_rn10, mdzg_kquad_rn12, mdzg_kquad_rn14, mdzg_kquad_rn16,
     mdzg_kquad_rn20, mdzg_kquad_rn24, mdzg_kquad_rn28, mdzg_kquad_rn32,
 };
@@ -86,7 +78,8 @@ static void lookup(int kid, int form, const void** f)
         *f = nullptr;
         if (kid == 0 || (kid >= MDZG_KID_GMP0 && kid < MDZG_KID_GMP0 + MDZG_NGMP))
             return;
-        kquad_rn[class_of_kid(kid)]((kid - 1) & 1, &p, &sl);
+        if (kquad_rn[class_of_kid(kid)])
+            kquad_rn[class_of_kid(kid)]((kid - 1) & 1, &p, &sl);
         *f = form == 3 ? p : sl;
         return;
     }

@@ -1175,11 +1175,11 @@ MP_HD void add_rn(mp<N>& r, const mp<N>& a_in, const mp<N>& b_in, uint32_t flipb
        than the quarter), so RN_p(A - B) = A.  Near the real axis wim2 is
        that small against wre2 in every iteration, and the squares'
        difference skips its alignment, carry chain and rounding.  Only the
-       squares' difference, only from 6 words (the vote in every addition of
-       the 4-word loop cost config 2 4 %) and only in the word-aligned
-       kernels (WORD_ALIGNED: p = 32N), whose register budget it leaves as
-       it was; the ragged 8- and 16-word kernels spilled more with it. */
-    if constexpr (SUBNN && WORD_ALIGNED && N >= 6) {
+       squares' difference, only where the loop is this one (from 12 words;
+       step_fast below) and only in the word-aligned kernels (WORD_ALIGNED:
+       p = 32N), whose register budget it leaves as it was; the ragged
+       16-word kernel spilled more with it. */
+    if constexpr (SUBNN && WORD_ALIGNED && N >= 12) {
         if (wave_all(d >= 32u * N + 2u)) {
 #pragma unroll
             for (int j = 0; j < N; ++j) r.m[j] = A[j];
