@@ -382,29 +382,35 @@ static double iteration_cycles(int kid)
    and with more classes than two rounds of the device's four queues at 1.45
    (36 tiles of 9 classes, 1.7: 27 ms with four lanes, 22.8 without).
 
-   SPREAD: past 1.9 the slowest class goes first, too, its blocks no two to a
-   CU while there are CUs for all.  In the order of kernel ids the wide classes
-   start last, on a chip that the others have filled unevenly, two blocks to a
-   CU: 60 tiles of 9 classes 39 ms by ids, 29 so; 14 tiles of 128x128 at 300 to
+   SPREAD: past 1.9 the slowest class goes first, too, if it has at most a block
+   a CU, and no two of its blocks go to one CU.  In the order of kernel ids the
+   wide classes start last, on a chip that the others have filled unevenly, two
+   blocks to a CU: 60 tiles of 9 classes 39 ms by ids, 29 so; 14 tiles of 128x128 at 300 to
    1000 bits 38.7 and 34.  First without the spread, a launch that comes a
    tenth of a millisecond after the other queues' ends up the same way: 30
    tiles of 6 classes 22 or 35 ms.
 
-   Between the lines the order of ids is the safer one (36 tiles 22.8 ms,
-   slowest first 22 or 34). */
+   A slowest class of more blocks than CUs fills the chip by itself, and first
+   it keeps the others waiting: 256 tiles of 64x64 to 512x512 pixels at 64 to
+   1024 bits, 79 % of whose work is the 1024-bit class, take 13.9 s by ids, 16.9
+   slowest first.  Between the lines, too, the order of ids is the safer one (36
+   tiles 22.8 ms, slowest first 22 or 34). */
 int mdzg_plan_batch(const mdzg_plan_tile* t, int n, int ncu, int* kids, int* how)
 {
     uint64_t pixels[MDZG_NKERNELS] = { 0 };
     double most[MDZG_NKERNELS] = { 0.0 };
     double slowest = 0.0, load = 0.0;
-    int nkid = 0;
+    int nkid = 0, first = 0;
     for (int i = 0; i < n; ++i)
         pixels[t[i].kid] += t[i].pixels;
     for (int i = 0; i < n; ++i) {
         const int kid = t[i].kid;
         const double c = (double)t[i].depth * iteration_cycles(kid);
         most[kid] = c > most[kid] ? c : most[kid];
-        slowest = c > slowest ? c : slowest;
+        if (c > slowest) {
+            slowest = c;
+            first = kid;
+        }
         load += (mdzg_dev_quad_pays(kid, pixels[kid], ncu) ? 2.0 : 1.0) * c * (double)t[i].pixels;
     }
     int classes = 0;
@@ -413,7 +419,7 @@ int mdzg_plan_batch(const mdzg_plan_tile* t, int n, int ncu, int* kids, int* how
     load /= slowest * 256.0 * (double)ncu;
     /* a class alone has no others to share with */
     *how = classes == 1 || load <= (classes <= 8 ? 1.9 : 1.45) ? MDZG_PLAN_FOUR
-           : load > 1.9                                         ? MDZG_PLAN_SPREAD
+           : load > 1.9 && pixels[first] <= 256u * (uint64_t)ncu ? MDZG_PLAN_SPREAD
                                                                 : 0;
     for (;;) {
         int k = -1;

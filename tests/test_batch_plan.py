@@ -1,7 +1,7 @@
 """The launch plan of a batch (mdzg_plan_batch): four lanes a pixel and the class
 whose pixels can take longest first while the batch leaves SIMDs idle; that class
-first and spread over the CUs where the load is high; the order of kernel ids
-between.  And batches of each kind against their tiles rendered alone.
+first and spread over the CUs where the load is high and it does not fill the
+chip itself; the order of kernel ids otherwise.  And batches of each kind against their tiles rendered alone.
 Tolerance: none."""
 import ctypes
 
@@ -37,9 +37,13 @@ SHEET = [(0, 1000, 96 * 96), (_k(128), 2500, 64 * 64), (_k(64), 1000, 64 * 64),
          (_k(320), 2000, 64 * 64), (_k(1024), 3600, 96 * 96)]
 
 
-@pytest.mark.parametrize("copies, how", [(1, FOUR), (30, SPREAD)])
-def test_slowest_class_first_at_low_and_high_load(copies, how):
-    kids, got = _plan(SHEET * copies)
+# the same with a 1024-bit tile so small that 28 of them have a block a CU at most
+SPARSE = [t if t[0] != _k(1024) else (t[0], t[1], 48 * 48) for t in SHEET]
+
+
+@pytest.mark.parametrize("tiles, copies, how", [(SHEET, 1, FOUR), (SPARSE, 28, SPREAD)])
+def test_slowest_class_first_at_low_and_high_load(tiles, copies, how):
+    kids, got = _plan(tiles * copies)
     assert got == how
     assert kids[0] == _k(1024) and kids[-1] == 0
     assert sorted(kids) == sorted({t[0] for t in SHEET})
@@ -47,17 +51,25 @@ def test_slowest_class_first_at_low_and_high_load(copies, how):
     assert kids.index(_k(512)) < kids.index(_k(256)) < kids.index(_k(64))
 
 
+@pytest.mark.parametrize("tiles", [SPARSE * 29, SHEET * 30, SHEET * 32])
+def test_a_slowest_class_that_fills_the_chip_does_not_go_first(tiles):
+    # 65536 pixels are a block of one lane a pixel on each CU
+    assert sum(t[2] for t in tiles if t[0] == _k(1024)) > 256 * NCU
+    kids, how = _plan(tiles)
+    assert how == 0 and kids == sorted(kids)
+
+
 def test_many_classes_between_the_lines_go_by_id():
-    nine = SHEET + [(_k(700), 900, 64 * 64)]
+    nine = SPARSE + [(_k(700), 900, 64 * 64)]
     how = {}
-    for copies in range(1, 40):
+    for copies in range(1, 29):
         kids, h = _plan(nine * copies)
         assert kids == sorted(kids) if h == 0 else kids[0] == _k(1024)
         how[copies] = h
     seen = list(how.values())
     assert seen == sorted(seen, key=[FOUR, 0, SPREAD].index) and set(seen) == {FOUR, 0, SPREAD}
     # up to eight classes have no such range
-    assert {_plan(SHEET * c)[1] for c in range(1, 40)} == {FOUR, SPREAD}
+    assert {_plan(SPARSE * c)[1] for c in range(1, 29)} == {FOUR, SPREAD}
 
 
 def test_order_is_by_time_not_by_id():
