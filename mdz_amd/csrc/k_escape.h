@@ -1116,7 +1116,8 @@ __device__ __forceinline__ uint32_t rn_op_fast(rn_state<N>& s, mp<N>& x, int op,
     case MDZG_OPP_MUL:
         for (int i = 0; i < reps; ++i) {
             mp<N> z;
-            rare = mul_fast<N, true, false>(z, x, y, pr);
+            rare = 0;
+            mul_fast<N, true, false>(z, x, y, pr, rare);
             if (__builtin_expect((rare & all) != 0, 0))
                 mul_rn<N, false>(z, x, y, 0);
             x = z;
@@ -1125,7 +1126,8 @@ __device__ __forceinline__ uint32_t rn_op_fast(rn_state<N>& s, mp<N>& x, int op,
     case MDZG_OPP_SQR:
         for (int i = 0; i < reps; ++i) {
             mp<N> z;
-            rare = mul_fast<N, true, true>(z, x, x, pr);
+            rare = 0;
+            mul_fast<N, true, true>(z, x, x, pr, rare);
             if (__builtin_expect((rare & all) != 0, 0))
                 mul_rn<N, true>(z, x, x, 0);
             x = z;
@@ -1137,10 +1139,11 @@ __device__ __forceinline__ uint32_t rn_op_fast(rn_state<N>& s, mp<N>& x, int op,
             mp<N> z;
             aligned<N> a;
             uint32_t S = 0;
+            rare = 0;
             align_fast<N>(a, x, cr);
             if ((lanes_of(is_far<N>(a)) & all) != 0)
                 align_far<N>(a, S, all);
-            rare = sum_fast<N, true, false>(z, a, x.s, cr.s ^ ((uint32_t)i & 1u), S, pr);
+            sum_fast<N, true, false>(z, a, x.s, cr.s ^ ((uint32_t)i & 1u), S, pr, rare);
             if (__builtin_expect((rare & all) != 0, 0)) {
                 add_rn<N>(z, x, cr, (uint32_t)i & 1u, 0);
                 clamp_zero<N>(z);
@@ -1153,10 +1156,11 @@ __device__ __forceinline__ uint32_t rn_op_fast(rn_state<N>& s, mp<N>& x, int op,
             mp<N> z;
             aligned<N> a;
             uint32_t S = 0;
+            rare = 0;
             align_fast<N>(a, s.wre2, s.wim2);
             if ((lanes_of(is_far<N>(a)) & all) != 0)
                 align_far<N>(a, S, all);
-            rare = sum_fast<N, true, true>(z, a, 0u, 1u, S, pr);
+            sum_fast<N, true, true>(z, a, 0u, 1u, S, pr, rare);
             if (__builtin_expect((rare & all) != 0, 0)) {
                 add_rn<N, SUB_NONNEG>(z, s.wre2, s.wim2, 1u, 0);
                 clamp_zero<N>(z);
@@ -1167,6 +1171,7 @@ __device__ __forceinline__ uint32_t rn_op_fast(rn_state<N>& s, mp<N>& x, int op,
         break;
     case MDZG_OPP_ESC:
         for (int i = 0; i < reps; ++i) {
+            rare = 0;
             h += (uint32_t)escaped_fast<N, true>(s.wim2, s.wre2, pr, rare) + (uint32_t)rare;
             asm volatile("" : "+v"(s.wim2.m[N - 1]));
         }

@@ -510,10 +510,10 @@ MP_HD void round_half(uint32_t& R0, uint32_t& R1, uint32_t half, uint32_t keep, 
 #endif
 }
 
-/* r = RN_p(a * b) (SQR: a * a); returns the lanes whose result may be wrong.
-   r may not be a or b. */
+/* r = RN_p(a * b) (SQR: a * a); rare: lanes whose result may be wrong.  r
+   may not be a or b. */
 template <int N, bool FULL, bool SQR>
-MP_HD lanes mul_fast(mp<N>& r, const mp<N>& a, const mp<N>& b, const rn_prec<FULL>& pr)
+MP_HD void mul_fast(mp<N>& r, const mp<N>& a, const mp<N>& b, const rn_prec<FULL>& pr, lanes& rare)
 {
     constexpr int K0 = short_col<N>();
     uint32_t H[N + 1];
@@ -533,19 +533,19 @@ MP_HD lanes mul_fast(mp<N>& r, const mp<N>& a, const mp<N>& b, const rn_prec<FUL
         constexpr uint32_t U = 2u * N;
         if constexpr (FULL) {
             round_gt(H[1], H[0], 0x7fffffffu, d, (int32_t)0x80000000u, H[0], s, sa, sb, co);
-            co = join(co, lanes_of((uint32_t)d < U));
+            rare = join(rare, lanes_of((uint32_t)d < U));
         } else {
             uint32_t y;
             round_half(H[1], H[2], pr.half, pr.keep, y, H[0], U - 1u, co);
             s = sa ^ sb;
-            co = join(co, lanes_of(y < U));
+            rare = join(rare, lanes_of(y < U));
         }
     }
+    rare = join(rare, co);
 #pragma unroll
     for (int j = 0; j < N; ++j) r.m[j] = H[j + 1];
     r.e = e;
     r.s = SQR ? 0u : s;
-    return co;
 }
 
 /* N words of v, shifted right by sh (mod 32), into N+1 words */
@@ -622,10 +622,7 @@ MP_HD void align_far(aligned<N>& x, uint32_t& S, lanes live)
 {
     constexpr uint32_t MOST = 32u * (N + 1);
     const bool fa = x.da > x.db;
-    /* not the lanes outside live, whose distances are any: a zero c is far from
-       every operand, and beside lanes that have escaped its wave shifted by
-       every stage in every iteration */
-    const uint32_t d = sel_mask(live, 0u, fa ? x.da : x.db);
+    const uint32_t d = fa ? x.da : x.db;
     const bool any = (lanes_of(fa) & live) != 0;
     uint32_t X[N + 1];
 #pragma unroll
@@ -661,11 +658,10 @@ MP_HD uint32_t lead_zeros(uint32_t x)
 }
 
 /* r = RN_p(a + b) of the aligned operands x with signs sa and sb (NONNEG: a - b
-   of nonnegative values), S a sticky bit of the smaller; returns rare lanes as
-   mul_fast */
+   of nonnegative values), S a sticky bit of the smaller; rare as in mul_fast */
 template <int N, bool FULL, bool NONNEG>
-MP_HD lanes sum_fast(mp<N>& r, aligned<N>& x, uint32_t sa, uint32_t sb, uint32_t S,
-                     const rn_prec<FULL>& pr)
+MP_HD void sum_fast(mp<N>& r, aligned<N>& x, uint32_t sa, uint32_t sb, uint32_t S,
+                    const rn_prec<FULL>& pr, lanes& rare)
 {
     const bool lt = x.A[N] < x.B[N];
     const uint32_t sub = NONNEG ? 1u : (sa ^ sb);
@@ -678,7 +674,7 @@ MP_HD lanes sum_fast(mp<N>& r, aligned<N>& x, uint32_t sa, uint32_t sb, uint32_t
     sum_chain<N + 1>(x.A, x.B, mA, mB, c);
     uint32_t* T = x.A;
     /* 0 or, where the top words were equal, negative: not decided here */
-    const lanes low = lanes_of((int32_t)T[N] <= 0);
+    rare = join(rare, lanes_of((int32_t)T[N] <= 0));
     const uint32_t lz = lead_zeros(T[N]);
     const uint32_t sh = 32u - lz;
     uint32_t R[N];
@@ -687,9 +683,9 @@ MP_HD lanes sum_fast(mp<N>& r, aligned<N>& x, uint32_t sa, uint32_t sb, uint32_t
     const uint32_t G = T[0] << (lz & 31u);
     lanes co;
     round_fast<N, FULL>(R, G, S, pr, r.e, x.e, lz, r.s, NONNEG ? 0u : sa, mA & 1u, co);
+    rare = join(rare, co);
 #pragma unroll
     for (int j = 0; j < N; ++j) r.m[j] = R[j];
-    return join(low, co);
 }
 
 /* RN_p(wim2 + wre2) > 4, decided from the top words in units of 2^-27 (each
@@ -707,7 +703,7 @@ MP_HD lanes escaped_fast(const mp<N>& wim2, const mp<N>& wre2, const rn_prec<FUL
     uint32_t thr = 1u << 29;
     if (!FULL && N == 1)          /* p >= 30 otherwise: less than a unit */
         thr += (1u << 29) >> ((32u - (uint32_t)kclr_of(pr)) & 31u);
-    unsure = lanes_of(est - thr + 4u <= 8u);
+    unsure = join(unsure, lanes_of(est - thr + 4u <= 8u));
     return lanes_of(est > thr);
 }
 
@@ -734,29 +730,18 @@ MP_HD void clamp_zero(mp<N>& v)
    live: z and z^2 advance; returns the lanes that escape.  The
    votes: one for the alignment distances of the first two sums, one for
    their and the product's rare lanes, one for the distance of the third sum,
-   one for everything after it.
-
-   Past a vote on rare lanes only what such a lane found rare is done again,
-   and not what a zero did: on the real axis (wim and c_im zeros) the product,
-   wim's sum and its square call every iteration rare, though what they leave
-   is a zero but for the sum's exponent and sign.  Orbits at fixed points on
-   the grid of the pixels cancel one sum in every iteration.  Square frames
-   about 0 hold such pixels: 256x256 of the set at 64, 80, 128 and 240 bits
-   took 0.69, 1.49, 1.10 and 2.74 ms where everything was done again, and take
-   0.46, 0.92, 0.93 and 1.83 so; of the Julia set of c = -3/4, whose column
-   re = 0 falls on the axis, 0.78, 1.42, 1.08 and 2.48, and 0.47, 0.61, 0.64
-   and 0.98. */
+   one for everything after it. */
 template <int N, bool FULL>
 MP_HD lanes step_fast(mp<N>& wre, mp<N>& wim, mp<N>& wre2, mp<N>& wim2, const mp<N>& cre,
                      const mp<N>& cim, const rn_form& f, const rn_prec<FULL>& pr, int32_t wz,
                      lanes live)
 {
     mp<N> t, u, w;
-    lanes rare_t, rare_w, rare_u, any;
+    lanes rare = 0;
     uint32_t su = 0, sw = 0;
     {
         aligned<N> xu, xw;
-        rare_t = mul_fast<N, FULL, false>(t, wre, wim, pr);        /* t1 = wre * wim   */
+        mul_fast<N, FULL, false>(t, wre, wim, pr, rare);           /* t1 = wre * wim   */
         t.e += 1;                                                  /* t1 *= 2          */
         t.s &= f.bs;                                               /* Burning Ship     */
         align_fast<N>(xu, wre2, wim2);
@@ -766,25 +751,20 @@ MP_HD lanes step_fast(mp<N>& wre, mp<N>& wim, mp<N>& wre2, mp<N>& wim2, const mp
             if ((lanes_of(is_far<N>(xu)) & live) != 0) align_far<N>(xu, su, live);
             if ((lanes_of(is_far<N>(xw)) & live) != 0) align_far<N>(xw, sw, live);
         }
-        rare_u = sum_fast<N, FULL, true>(u, xu, 0u, 1u, su, pr);   /* t1 = wre2 - wim2 */
-        any = join(rare_t, rare_u);
-        rare_w = sum_fast<N, FULL, false>(w, xw, t.s, cim.s, sw, pr);  /* wim = t1 + c_im */
+        sum_fast<N, FULL, true>(u, xu, 0u, 1u, su, pr, rare);      /* t1 = wre2 - wim2 */
+        sum_fast<N, FULL, false>(w, xw, t.s, cim.s, sw, pr, rare); /* wim = t1 + c_im  */
     }
-    if (__builtin_expect((join(any, rare_w) & live) != 0, 0)) {
-        const bool axis = is_zero<N>(wim) & is_zero<N>(cim);
-        if (((rare_t | rare_w) & live & ~lanes_of(axis)) != 0) {
-            mul_rn<N, false>(t, again(wre), again(wim), kclr_of(pr));
-            t.e += 1;
-            t.s &= f.bs;
-            add_rn<N>(w, t, again(cim), 0u, kclr_of(pr));
-        }
+    if (__builtin_expect((rare & live) != 0, 0)) {
+        mul_rn<N, false>(t, again(wre), again(wim), kclr_of(pr));
+        t.e += 1;
+        t.s &= f.bs;
+        add_rn<N>(w, t, again(cim), 0u, kclr_of(pr));
+        add_rn<N, SUB_NONNEG>(u, again(wre2), again(wim2), 1u, kclr_of(pr));
         clamp_zero<N>(w);
-        if ((rare_u & live) != 0)
-            add_rn<N, SUB_NONNEG>(u, again(wre2), again(wim2), 1u, kclr_of(pr));
     }
     u.s &= f.ce ^ ((uint32_t)wz & f.va);                           /* Celtic           */
     wim = w;
-    lanes rare_r;
+    lanes rare2 = 0;
     uint32_t sr = 0;
     {
         aligned<N> xr;
@@ -792,26 +772,18 @@ MP_HD lanes step_fast(mp<N>& wre, mp<N>& wim, mp<N>& wre2, mp<N>& wim2, const mp
         const lanes far = lanes_of(is_far<N>(xr)) & live;
         if (far != 0)
             align_far<N>(xr, sr, live);
-        rare_r = sum_fast<N, FULL, false>(wre, xr, u.s, cre.s, sr, pr);    /* wre = t1 + c_re */
+        sum_fast<N, FULL, false>(wre, xr, u.s, cre.s, sr, pr, rare2);  /* wre = t1 + c_re */
     }
-    const lanes rare_im = mul_fast<N, FULL, true>(wim2, wim, wim, pr);     /* wim2 = wim^2 */
-    any = join(rare_r, rare_im);
-    const lanes rare_re = mul_fast<N, FULL, true>(wre2, wre, wre, pr);     /* wre2 = wre^2 */
-    any = join(any, rare_re);
-    lanes unsure;
-    lanes esc = escaped_fast<N, FULL>(wim2, wre2, pr, unsure);
-    if (__builtin_expect((join(any, unsure) & live) != 0, 0)) {
-        const lanes im = rare_im & ~lanes_of(is_zero<N>(wim));
-        if (((rare_r | rare_re | unsure | im) & live) != 0) {
-            add_rn<N>(wre, again(u), again(cre), 0u, kclr_of(pr));
-            clamp_zero<N>(wre);
-            /* up to 5 words the loop pays more for a choice here (moves) */
-            if (N < 6 || (im & live) != 0)
-                mul_rn<N, true>(wim2, again(wim), wim, kclr_of(pr));
-            mul_rn<N, true>(wre2, again(wre), wre, kclr_of(pr));
-            const double thresh = 4.0 + ldexp(1.0, 2 - (32 * N - kclr_of(pr)));
-            esc = lanes_of(escaped<N>(wim2, wre2, thresh, kclr_of(pr)));
-        }
+    mul_fast<N, FULL, true>(wim2, wim, wim, pr, rare2);            /* wim2 = wim^2     */
+    mul_fast<N, FULL, true>(wre2, wre, wre, pr, rare2);            /* wre2 = wre^2     */
+    lanes esc = escaped_fast<N, FULL>(wim2, wre2, pr, rare2);
+    if (__builtin_expect((rare2 & live) != 0, 0)) {
+        add_rn<N>(wre, again(u), again(cre), 0u, kclr_of(pr));
+        clamp_zero<N>(wre);
+        mul_rn<N, true>(wim2, again(wim), wim, kclr_of(pr));
+        mul_rn<N, true>(wre2, again(wre), wre, kclr_of(pr));
+        const double thresh = 4.0 + ldexp(1.0, 2 - (32 * N - kclr_of(pr)));
+        esc = lanes_of(escaped<N>(wim2, wre2, thresh, kclr_of(pr)));
     }
     return esc;
 }
