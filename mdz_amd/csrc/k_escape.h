@@ -72,17 +72,19 @@ __device__ __forceinline__ int read_cancel(const volatile int* p)
     return *(g_cflag*)p;
 }
 
-/* Rounds between two reads of the cancel flag, less 1: 15, fewer where the chunk
-   would make them more than MOST iterations, so that a long chunk does not
-   make a cancelled job run on.  512 iterations up to 10 words (0.7 ms at 128
-   bits; a read waits for the count stores before it, and every 128 iterations
-   cost frames of quickly escaping pixels 5 to 15 % at 80 bits), 128 for wider
-   ones (1.2 ms at 512 bits). */
-template <int MOST>
+/* Rounds between two reads of the cancel flag, less 1, in the loops from 12 words
+   and the four-lane ones: 15, fewer where the chunk would make them more than
+   128 iterations (1.2 ms at 512 bits), so that a long chunk does not make a
+   cancelled job run on.  Up to 10 words it is 15, a constant, and a launch's
+   chunk at most 32 (launch.hip): 512 iterations, 0.7 ms at 128 bits.  The
+   mask in a register cost those loops 1 % and a 640x480 frame at 128 bits
+   whose pixels escape 19 % (12.1 -> 14.4 ms), 128 iterations frames of quickly
+   escaping pixels 5 to 15 % at 80 bits. */
+template <int N>
 __device__ __forceinline__ uint32_t cancel_mask(int chunk)
 {
     /* >=: with <= the compiler holds the steps in vector registers */
-    return chunk >= MOST ? 0u : (chunk >= MOST / 2 ? 1u : (chunk >= MOST / 4 ? 3u : (chunk >= MOST / 8 ? 7u : 15u)));
+    return N < 12 ? 15u : chunk >= 128 ? 0u : (chunk >= 64 ? 1u : (chunk >= 32 ? 3u : (chunk >= 16 ? 7u : 15u)));
 }
 
 /* Queue slots are claimed per wave.  A wave whose lanes need n slots takes
@@ -1304,7 +1306,7 @@ __global__ __launch_bounds__(256, (rn_min_waves<N, FULL>())) void k_rn_persist(c
     bool active = false;
     int fractal = 0, kclr = 0;
     uint32_t round = 0;
-    const uint32_t often = cancel_mask<(N < 12 ? 512 : 128)>(chunk);
+    const uint32_t often = cancel_mask<N>(chunk);
     int32_t wz = 0, depth = 0;
     uint32_t* out = nullptr;
     __shared__ uint32_t c_lds[c_in_lds<N>() ? 2 * (N + 2) * 256 : 1];

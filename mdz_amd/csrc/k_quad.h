@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256, 2) void k_rn_quad(const mdzg_dtile* tiles, int
     bool active = false, drained = false;
     int kclr = 0;
     uint32_t round = 0;
-    const uint32_t often = cancel_mask<128>(chunk);
+    const uint32_t often = cancel_mask<12>(chunk);
     int32_t wz = 0, depth = 0;
     uint32_t* out = nullptr;
     rn_form fm = { 1u, 1u, 0u };

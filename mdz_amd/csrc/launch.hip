@@ -244,6 +244,15 @@ int mdzg_dev_node_fill(mdzg_gnode* n, uint32_t* p, uint64_t count, uint32_t v)
     return 0;
 }
 
+/* The RN loops up to 10 words read the cancel flag every 16 chunks: with at most
+   32 iterations a chunk, every 512.  Nothing tuned is longer. */
+static int launch_chunk(int kid, int chunk)
+{
+    if (kid == 0 || (kid >= MDZG_KID_GMP0 && kid < MDZG_KID_GMP0 + MDZG_NGMP) || chunk <= 32)
+        return chunk;
+    return class_of_kid(kid) <= 8 /* 10 words */ ? 32 : chunk;
+}
+
 int mdzg_dev_node_persist(mdzg_gnode* n, int kid, const mdzg_dtile* d_tiles, int ntiles,
                           uint64_t total, unsigned long long* d_counter, const int* d_cancel,
                           int quad, int grid, int chunk)
@@ -254,6 +263,7 @@ int mdzg_dev_node_persist(mdzg_gnode* n, int kid, const mdzg_dtile* d_tiles, int
     lookup(kid, quad ? 3 : 1, &f);
     if (!f)
         return -1;
+    chunk = launch_chunk(kid, chunk);
     node_init(n, f, (unsigned)grid, 256);
     node_arg(n, d_tiles);
     node_arg(n, ntiles);
@@ -333,6 +343,7 @@ int mdzg_dev_launch_persist(int kid, const mdzg_dtile* d_tiles, int ntiles, uint
     lookup(kid, quad ? 3 : 1, &f);
     if (!f)
         return -1;
+    chunk = launch_chunk(kid, chunk);
     void* args[] = { (void*)&d_tiles, (void*)&ntiles, (void*)&total, (void*)&d_counter,
                      (void*)&d_cancel, (void*)&chunk };
     return hipLaunchKernel(f, dim3(grid), dim3(256), args, 0, st) == hipSuccess ? 0 : -3;
