@@ -269,7 +269,9 @@ __device__ __forceinline__ bool fp64_step_any(fp64_state& s, const fp64_form& f,
    seen when the distance to the kept z is a multiple of q: 60 is one for q =
    1..6, 10, 12, 15, 20 and 30.  The persistent kernel's runs keep one z a
    lane and replace it on all lanes at once, after 60, 120, 180, 240, 360 ...
-   iterations of the run: four instructions and a vote in about 600.  A lane
+   iterations of the run: four instructions and a vote in about 600 (a
+   1920x1080 frame of escaping pixels in the seahorse valley 0.521 -> 0.533
+   ms, of the whole set 0.517 -> 0.416).  A lane
    that starts a pixel forgets its z (a NaN, which no orbit but one of NaNs,
    never past the escape test either, equals). */
 #ifndef MDZG_CYCLE_FP64
@@ -739,8 +741,10 @@ __device__ __forceinline__ void load_mp(mp<N>& v, const uint32_t* p)
 
 /* minimum waves per SIMD the RN kernels are compiled for: small N keep
    several waves resident, large N share the register file by two (the ragged
-   32-word class, too, since its rounding masks only the cut's words: 1.35
-   times the pixel rate of one wave) */
+   32-word class, too, since its rounding masks only the cut's words: deep
+   views at 1000 bits take 0.69 to 0.84 of the time of this kernel with one
+   wave, overviews of 120,000 to 170,000 pixels, which two waves a SIMD hold
+   at once, 1.2 to 1.9 times it) */
 template <int N, bool FULL>
 constexpr int rn_min_waves()
 {

@@ -23,7 +23,9 @@
  * About 0.45 of the instructions in a lane's iteration, for four times the
  * lanes: 64x64 tiles at 300, 512 and 1024 bits take 1.18, 2.48 and 8.4 ms
  * against 1.95, 4.35 and 16.7 with one lane a pixel.  Up to 32768 pixels
- * (rule and figures: mdzg_dev_quad_pays).
+ * (rule and figures: mdzg_dev_quad_pays).  At that size every pixel of a
+ * launch has its quad where two blocks fit a CU, as they do: the persistent
+ * form then claims once, and only the slices refill.
  *
  * The loop's state between iterations: v = z (wim on q0, wre on q2) and p =
  * the products of z (2 t's product on q0, wim2 on q1, wre2 on q2).  A pixel

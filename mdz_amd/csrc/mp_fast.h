@@ -36,11 +36,25 @@
  *   128 bits   2928 -> 1718      135 -> 146
  *   176 bits   4369 -> 2279       89 -> 102
  *   256 bits   3967 -> 2740       83 -> 81 (frames of escaping pixels: 75 -> 78)
- * What is left is VALU issue: 301 instructions an iteration at 4 words, 39 of
- * them multiply-accumulates.  At 320 bits an iteration alone takes 3,300
- * cycles against 4,800 (a 480x360 frame of a saved scene 26.1 -> 21.3 ms); the
- * ragged 10-word kernel, whose cut may lie in the second word, and those from
- * 12 words up, where the products outweigh the votes, keep add_rn and mul_rn.
+ * What is left is VALU issue: 309 instructions an iteration at 4 words, 39 of
+ * them multiply-accumulates.  Where all lanes of a wave agree and the chip is
+ * full, the votes were the cheaper form at 6 and 8 whole words: 517
+ * instructions an iteration at 8 words against 541 here.  A 1920x1080 frame of
+ * orbits that settle too slowly to be found periodic (300 iterations) takes
+ * 5.9 ms at 192 bits and 7.9 at 256, with votes 5.7 and 7.1; frames with
+ * escaping pixels gain 2 to 39 %.  add_rn in the waves whose lanes agree took
+ * 6.6 and 8.0 ms.
+ * An exact zero is rare here: a wave with a pixel on the real axis does its
+ * iterations twice.  256x256 frames of the set, whose middle row lies there,
+ * take 1.06 (64 bits), 1.34 (80), 1.23 (128) and 1.27 (256) times what they took
+ * with votes; with that row elsewhere 0.5 to 0.7 times.  Telling zeros from rare
+ * lanes gave most of that back, but slowed other frames by up to 2 % and, by
+ * an uneven second round of waves, a 640x480 frame of escaping pixels at 128
+ * bits from 12.1 to 14.5 ms.
+ * At 320 bits an iteration alone takes 3,300 cycles against 4,800 (a 480x360
+ * frame of a saved scene 26.1 -> 21.3 ms); the ragged 10-word kernel, whose cut
+ * may lie in the second word, and those from 12 words up keep add_rn and
+ * mul_rn (this form was not measured there).
  *
  * A precision of p = 32N - kclr bits with 0 <= kclr < 32 is covered: rounding
  * at bit kclr of the lowest word is one add with carry and a mask.
