@@ -31,28 +31,30 @@ def _k(p, path=M.PATH_MPFR):
     return M.kernel_id(path, p)
 
 
-# a contact sheet: classes from FP64 to 1024 bits, the deepest the slowest
-SHEET = [(0, 1000, 96 * 96), (_k(128), 2500, 64 * 64), (_k(64), 1000, 64 * 64),
-         (_k(256), 2500, 96 * 96), (_k(256, M.PATH_GMP), 3000, 64 * 64), (_k(512), 1700, 64 * 64),
-         (_k(320), 2000, 64 * 64), (_k(1024), 3600, 96 * 96)]
+def _sheet(side=96):
+    """A contact sheet: classes from FP64 to 1024 bits, the deepest, of side^2 pixels,
+    the slowest.  Not made on import: the library must not load before torch, whose
+    HIP runtime would be a second one in the process."""
+    return [(0, 1000, 96 * 96), (_k(128), 2500, 64 * 64), (_k(64), 1000, 64 * 64),
+            (_k(256), 2500, 96 * 96), (_k(256, M.PATH_GMP), 3000, 64 * 64),
+            (_k(512), 1700, 64 * 64), (_k(320), 2000, 64 * 64), (_k(1024), 3600, side * side)]
 
 
-# the same with a 1024-bit tile so small that 28 of them have a block a CU at most
-SPARSE = [t if t[0] != _k(1024) else (t[0], t[1], 48 * 48) for t in SHEET]
-
-
-@pytest.mark.parametrize("tiles, copies, how", [(SHEET, 1, FOUR), (SPARSE, 28, SPREAD)])
-def test_slowest_class_first_at_low_and_high_load(tiles, copies, how):
+# 28 tiles of 48x48 have a block a CU at most
+@pytest.mark.parametrize("side, copies, how", [(96, 1, FOUR), (48, 28, SPREAD)])
+def test_slowest_class_first_at_low_and_high_load(side, copies, how):
+    tiles = _sheet(side)
     kids, got = _plan(tiles * copies)
     assert got == how
     assert kids[0] == _k(1024) and kids[-1] == 0
-    assert sorted(kids) == sorted({t[0] for t in SHEET})
+    assert sorted(kids) == sorted({t[0] for t in tiles})
     # 13.6M cycles at 512 bits, 6.9M at 256, 1.1M at 64
     assert kids.index(_k(512)) < kids.index(_k(256)) < kids.index(_k(64))
 
 
-@pytest.mark.parametrize("tiles", [SPARSE * 29, SHEET * 30, SHEET * 32])
-def test_a_slowest_class_that_fills_the_chip_does_not_go_first(tiles):
+@pytest.mark.parametrize("side, copies", [(48, 29), (96, 30), (96, 32)])
+def test_a_slowest_class_that_fills_the_chip_does_not_go_first(side, copies):
+    tiles = _sheet(side) * copies
     # 65536 pixels are a block of one lane a pixel on each CU
     assert sum(t[2] for t in tiles if t[0] == _k(1024)) > 256 * NCU
     kids, how = _plan(tiles)
@@ -60,7 +62,7 @@ def test_a_slowest_class_that_fills_the_chip_does_not_go_first(tiles):
 
 
 def test_many_classes_between_the_lines_go_by_id():
-    nine = SPARSE + [(_k(700), 900, 64 * 64)]
+    nine = _sheet(48) + [(_k(700), 900, 64 * 64)]
     how = {}
     for copies in range(1, 29):
         kids, h = _plan(nine * copies)
@@ -69,7 +71,7 @@ def test_many_classes_between_the_lines_go_by_id():
     seen = list(how.values())
     assert seen == sorted(seen, key=[FOUR, 0, SPREAD].index) and set(seen) == {FOUR, 0, SPREAD}
     # up to eight classes have no such range
-    assert {_plan(SPARSE * c)[1] for c in range(1, 29)} == {FOUR, SPREAD}
+    assert {_plan(_sheet(48) * c)[1] for c in range(1, 29)} == {FOUR, SPREAD}
 
 
 def test_order_is_by_time_not_by_id():
